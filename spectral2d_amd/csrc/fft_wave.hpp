@@ -1,19 +1,20 @@
 // fft_wave.hpp -- compile-time Stockham FFT on a lane group.
 //
 // A length n = E*TG transform (n = 2^a 3^b) is carried by a group of TG
-// lanes (TG a power of two, 2..256). Groups of up to 64 lanes live inside
-// one wave (64/TG groups per wave); larger groups span TG/64 waves of one
+// lanes, TG a power of two (2..256) or, with E = 12, 3*2^k (6..192). Groups
+// that divide a wave live inside one (64/TG groups per wave); the others
+// (TG > 64, or 3*2^k lanes, whose groups straddle waves) span waves of one
 // workgroup. Lane t of the group holds x[t + TG*s], s < E. The early passes
-// are radix-R Stockham passes (R in {8, 4, 2}, R | E, the radices multiply
-// to TG) that exchange through the group's LDS slice; the final pass is one
-// radix-E butterfly per lane, in registers, whose outputs X[t + TG*m] are
-// again the lane's own elements.
+// are radix-R Stockham passes (R in {12, 8, 6, 4, 2}, R | E, the radices
+// multiply to TG) that exchange through the group's LDS slice; the final
+// pass is one radix-E butterfly per lane, in registers, whose outputs
+// X[t + TG*m] are again the lane's own elements.
 //
-// LDS slots are permuted inside aligned blocks of 16 elements (LdsPad), which
-// spreads the strided Stockham writes and the contiguous reads over the
-// banks without padding. Groups inside one wave synchronise with wave-scope fences;
-// multi-wave groups use workgroup barriers, which every thread of the
-// workgroup must reach the same number of times.
+// LDS slots are spread over the banks (LdsMap): for a power of two by a
+// permutation inside aligned blocks of 16 elements, without padding; for
+// 3*2^k by one pad element in 12. Groups inside one wave synchronise with
+// wave-scope fences; the others use workgroup barriers, which every thread
+// of the workgroup must reach the same number of times.
 //
 // Per-lane twiddles come from the FP64-generated table tw[e] =
 // exp(-2 pi i e / n) of the transform length (rounded to T); the twiddles
@@ -36,32 +37,41 @@ __device__ __forceinline__ void wave_sync()
 template <int TG>
 __device__ __forceinline__ void group_sync()
 {
-    if constexpr (TG > 64)
+    if constexpr (64 % TG != 0)
         __syncthreads();
     else
         wave_sync();
 }
 
-// LDS slot of element i: bits 0-3 XORed with bits 3-6, a permutation inside
-// each aligned block of 16 elements (n is a multiple of 16 for every size
-// used). It keeps the strided Stockham writes and the contiguous reads
-// within 1.25-1.5x of conflict-free for both 32- and 64-bank LDS, with no
-// padding.
+// LDS slot of element i of a TG-lane group.
 //
-// Every exchange addresses slot b + c of a lane-dependent b and a constant c
-// that share no set bit. idx distributes over such sums as idx(b) ^ idx(c),
-// and as it only changes bits 0-3 that is (idx(b) ^ (idx(c) & 15)) +
-// (c & ~15): with idx(b) computed once per pass, an access costs one XOR
-// with a constant, and the addition folds into the LDS instruction's offset.
-template <typename T>
-struct LdsPad {
-    static __host__ __device__ constexpr int idx(int i) { return i ^ ((i >> 3) & 15); }
-    // idx(b + c) from ib = idx(b), for b & c == 0
+// TG a power of two: bits 0-3 XORed with bits 3-6, a permutation inside each
+// aligned block of 16 elements (n is a multiple of 16 for every size used).
+// It keeps the strided Stockham writes and the contiguous reads within
+// 1.25-1.5x of conflict-free for both 32- and 64-bank LDS, with no padding.
+// Every exchange addresses slot b + c, with b from the lane and c a
+// compile-time constant that shares no set bit with b, so that idx_sum takes
+// one XOR with a constant, and the addition folds into the LDS instruction's
+// offset.
+//
+// TG = 3*2^k: i + i/12. The first pass (radix 12, or 6 for TG = 6) writes R
+// consecutive elements per lane, 13 slots apart (a stride of 12 would put
+// every fourth lane of an FP64 write, every eighth of an FP32 one, on the
+// same banks), and every later offset is a multiple of 12: idx(b + c) is
+// idx(b) + idx(c), all of it in the instruction's offset.
+template <int TG>
+struct LdsMap {
+    static constexpr bool P2 = (TG & (TG - 1)) == 0;
+    static __host__ __device__ constexpr int idx(int i)
+    {
+        return P2 ? i ^ ((i >> 3) & 15) : i + i / 12;
+    }
+    // idx(b + c) from ib = idx(b), for the b and c of the exchanges
     static __host__ __device__ constexpr int idx_sum(int ib, int c)
     {
-        return (ib ^ (idx(c) & 15)) + (c & ~15);
+        return P2 ? (ib ^ (idx(c) & 15)) + (c & ~15) : ib + idx(c);
     }
-    static constexpr int size(int n) { return n; }
+    static constexpr int size(int n) { return P2 ? n : n / 12 * 13; }
 };
 
 // idx_sum against idx over every pair of disjoint 8-bit values (idx reads
@@ -70,12 +80,57 @@ constexpr bool lds_idx_sum_exact()
 {
     for (int b = 0; b < 256; ++b)
         for (int c = 0; c < 256; ++c)
-            if ((b & c) == 0 && LdsPad<float>::idx_sum(LdsPad<float>::idx(b), c) !=
-                                    LdsPad<float>::idx(b + c))
+            if ((b & c) == 0 && LdsMap<1>::idx_sum(LdsMap<1>::idx(b), c) != LdsMap<1>::idx(b + c))
                 return false;
     return true;
 }
 static_assert(lds_idx_sum_exact(), "idx_sum differs from idx");
+
+// Largest early radix in {12, 6, 8, 4, 2} dividing both E and the remaining
+// product rem of the group size (12 and 6 only serve TG = 3*2^k: they take
+// its factor 3 in the first pass).
+constexpr int early_radix(int E, int rem)
+{
+    return (E % 12 == 0 && rem % 12 == 0) ? 12
+           : (E % 6 == 0 && rem % 6 == 0) ? 6
+           : (E % 8 == 0 && rem % 8 == 0) ? 8
+           : (E % 4 == 0 && rem % 4 == 0) ? 4
+                                          : 2;
+}
+
+// The same for TG = 3*2^k and E = 12, over every address of its transform:
+// the reads t + TG s and each early pass's writes (t - k) R + k + TG q R + m Ls.
+template <int TG>
+constexpr bool lds_idx_sum_exact3()
+{
+    using M = LdsMap<TG>;
+    constexpr int E = 12;
+    for (int t = 0; t < TG; ++t) {
+        for (int s = 0; s < E; ++s)
+            if (M::idx_sum(M::idx(t), TG * s) != M::idx(t + TG * s)) return false;
+        for (int Ls = 1; Ls < TG;) {
+            const int R = early_radix(E, TG / Ls), k = t % Ls, b = (t - k) * R + k;
+            for (int q = 0; q < E / R; ++q)
+                for (int m = 0; m < R; ++m)
+                    if (M::idx_sum(M::idx(b), TG * q * R + m * Ls) !=
+                        M::idx(b + TG * q * R + m * Ls))
+                        return false;
+            Ls *= R;
+        }
+    }
+    return true;
+}
+static_assert(lds_idx_sum_exact3<6>() && lds_idx_sum_exact3<12>() && lds_idx_sum_exact3<24>() &&
+                  lds_idx_sum_exact3<48>() && lds_idx_sum_exact3<96>() && lds_idx_sum_exact3<192>(),
+              "idx_sum differs from idx");
+
+// t % Ls for a lane index t >= 0.
+template <int Ls>
+__device__ __forceinline__ int lane_mod(int t)
+{
+    if constexpr ((Ls & (Ls - 1)) == 0) return t & (Ls - 1);
+    else return (int)((unsigned)t % (unsigned)Ls);
+}
 
 // Compile-time loop: f(std::integral_constant<int, I>) for I in [B, N).
 template <int B, int N, typename F>
@@ -158,13 +213,6 @@ __device__ __forceinline__ void dft_ct(cpx<T> *a)
     }
 }
 
-// Largest early radix in {8, 4, 2} dividing both E and the remaining
-// product rem of the group size.
-constexpr int early_radix(int E, int rem)
-{
-    return (E % 8 == 0 && rem % 8 == 0) ? 8 : (E % 4 == 0 && rem % 4 == 0) ? 4 : 2;
-}
-
 // Number of per-lane twiddles of the early passes before the one at Ls
 // (the first pass, Ls = 1, needs none).
 template <int E, int TG, int Ls, int L = 1>
@@ -219,7 +267,7 @@ struct GroupTw {
     __device__ __forceinline__ cpx<T> early(int m) const
     {
         if constexpr (PE) return e[early_tw_offset<E, TG, Ls>() + m - 1];
-        else return tw[m * (t & (Ls - 1)) * (n / (Ls * R))];
+        else return tw[m * lane_mod<Ls>(t) * (n / (Ls * R))];
     }
     // twiddle m (1 <= m < E) of the final pass
     __device__ __forceinline__ cpx<T> final(int m) const
@@ -236,7 +284,7 @@ struct GroupTw {
             constexpr int R = early_radix(E, TG / Ls);
             if constexpr (Ls > 1) {
                 constexpr int o = early_tw_offset<E, TG, Ls>(), ts = n / (Ls * R);
-                const int k = t & (Ls - 1);
+                const int k = lane_mod<Ls>(t);
 #pragma unroll
                 for (int m = 1; m < R; ++m) e[o + m - 1] = tw[m * k * ts];
             }
@@ -259,10 +307,10 @@ template <typename T, int E, int TG, int R, int Ls, int D, class G>
 __device__ __forceinline__ void group_pass(cpx<T> (&v)[E], cpx<T> *lds, int t, const G &g)
 {
     constexpr int Q = E / R;
-    const int k = t & (Ls - 1);
+    const int k = lane_mod<Ls>(t);
     // slot of output m of butterfly q: (t - k) R + k, the lane's part, plus
     // TG q R + m Ls, which shares no bit with it
-    const int ib = LdsPad<T>::idx((t - k) * R + k);
+    const int ib = LdsMap<TG>::idx((t - k) * R + k);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         cpx<T> a[R];
@@ -272,9 +320,9 @@ __device__ __forceinline__ void group_pass(cpx<T> (&v)[E], cpx<T> *lds, int t, c
 #pragma unroll
             for (int m = 1; m < R; ++m) a[m] = mul(a[m], dir<T, D>(g.template early<Ls, R>(m)));
         }
-        dft<T, R, D>(a);
+        dft_ct<T, R, D>(a);
 #pragma unroll
-        for (int m = 0; m < R; ++m) lds[LdsPad<T>::idx_sum(ib, TG * q * R + m * Ls)] = a[m];
+        for (int m = 0; m < R; ++m) lds[LdsMap<TG>::idx_sum(ib, TG * q * R + m * Ls)] = a[m];
     }
 }
 
@@ -286,9 +334,9 @@ __device__ __forceinline__ void early_passes(cpx<T> (&v)[E], cpx<T> *lds, int t,
         static_assert(E % R == 0 && (TG / Ls) % R == 0, "no early radix");
         group_pass<T, E, TG, R, Ls, D, G>(v, lds, t, g);
         group_sync<TG>();
-        const int it = LdsPad<T>::idx(t);
+        const int it = LdsMap<TG>::idx(t);
 #pragma unroll
-        for (int s = 0; s < E; ++s) v[s] = lds[LdsPad<T>::idx_sum(it, TG * s)];
+        for (int s = 0; s < E; ++s) v[s] = lds[LdsMap<TG>::idx_sum(it, TG * s)];
         group_sync<TG>();
         early_passes<T, E, TG, D, Ls * R, G>(v, lds, t, g);
     }
@@ -316,7 +364,7 @@ __device__ __forceinline__ void final_pass(cpx<T> (&v)[E], const G &g)
 }
 
 // Full transform of the group: on entry v[s] = x[t + TG*s], on exit
-// v[s] = X[t + TG*s]. lds is the group's slice (LdsPad<T>::size(n)); g holds
+// v[s] = X[t + TG*s]. lds is the group's slice (LdsMap<TG>::size(n)); g holds
 // the lane's twiddles (GroupTw::load with the table of length n).
 template <typename T, int E, int TG, int D, int PRE>
 __device__ __forceinline__ void group_fft(cpx<T> (&v)[E], cpx<T> *lds, int t,

@@ -1,6 +1,7 @@
 // kernels_fused_v2.hpp -- the fused RK3 stage kernels on lane-group FFTs
 // (fft_wave.hpp), compiled for the padded sizes Np in {96, 192, 384, 768,
-// 1536, 3072}. Same mathematics and data layout as kernels_fused.hpp
+// 1536, 3072} (N a power of two) and {144, 288, 576, 1152, 2304} (N = 3*2^k).
+// Same mathematics and data layout as kernels_fused.hpp
 // (compact omega, mixed (kx, y) fields G/H); other sizes use those kernels.
 //
 // Elements per lane: 12 in both precisions (a 1536-point transform spans
@@ -58,16 +59,26 @@ template <typename T, int NP, int V = 0>
 struct WaveCfg {
     static constexpr int E = (V & VAR_E24) ? 24 : 12;
     static constexpr int TG = NP / E;
-    // lines (columns / rows) per block of passes A and B, LPB * TG threads
-    static constexpr int LPB_A = TG >= 256 ? (sizeof(T) == 4 ? 2 : 1) : 256 / TG;
+    static constexpr bool P2 = (TG & (TG - 1)) == 0; // else 3*2^k lanes
+    // lines (columns / rows) per block of passes A and B, LPB * TG threads.
+    // 3*2^k lanes: three waves per block, so that every block is whole waves
+    // (FP32 pass A: six, G rows in segments twice as long; 192 lanes: two
+    // columns, whose LDS two blocks still share a CU). What bounds these
+    // sizes is what bounds their neighbours: latency (one round of blocks) up
+    // to Np = 1152, the 256 MB cache and VALU issue at 2304. FP64 Np = 1152:
+    // 13, 21 and 10 us for A, B and C (26, 35 and 28 MB of algorithmic traffic)
+    static constexpr int THR3_A = sizeof(T) == 4 && TG > 12 ? 384 : 192;
+    static constexpr int LPB_A = !P2 ? (TG >= 192 ? 2 : THR3_A / TG)
+                                 : TG >= 256 ? (sizeof(T) == 4 ? 2 : 1) : 256 / TG;
     // pass B: two rows per lane group from Np = 1536 up (passB_pair)
     static constexpr bool PAIR_B = (NP >= 1536) != ((V & VAR_PAIR) != 0);
-    static constexpr int LPB_B = PAIR_B ? 2 : TG >= 128 && sizeof(T) == 8 ? 1 : TG >= 256 ? 2 : 256 / TG;
+    static constexpr int LPB_B = PAIR_B ? 2 : !P2 ? 192 / TG
+                                 : TG >= 128 && sizeof(T) == 8 ? 1 : TG >= 256 ? 2 : 256 / TG;
     static constexpr int THR_B = PAIR_B ? LPB_B * TG / 2 : LPB_B * TG; // lanes per block
-    // pass C: column groups per half, two halves per block
-    static constexpr int GPB = TG >= 64 ? 1 : 64 / TG;
-    static constexpr int BLK = TG >= 64 ? TG : 64; // threads per half
-    static constexpr int SLICE = LdsPad<T>::size(NP);
+    // pass C: column groups per half, two halves per block (whole waves each)
+    static constexpr int GPB = !P2 ? 192 / TG : TG >= 64 ? 1 : 64 / TG;
+    static constexpr int BLK = GPB * TG; // threads per half
+    static constexpr int SLICE = LdsMap<TG>::size(NP);
     // register budgets, waves per SIMD, of passes A and C (FP64 pass C: 256
     // VGPRs hold a transform's data, its twiddles and the loads issued ahead
     // of it without spills; FP64 pass A fits three waves in 168 by loading
@@ -81,8 +92,11 @@ struct WaveCfg {
     // final pass's as powers of W^t (FP64: 168 VGPRs, three waves per SIMD,
     // 7 % less time at Np = 1536; FP32 Np <= 768: five waves, 7 % less
     // time for the mixed ensemble)
+    // (FP64 3*2^k: all from the table, as accurate as the runtime plans' to
+    // 20 %; powers took 4 % off these passes and added to the error)
+    static constexpr bool TAB = !P2 && sizeof(T) == 8;
     static constexpr int TW_PRE_C0 =
-        sizeof(T) == 8 || TG <= 64 ? (TW_EARLY | TW_FINAL_POW) : TW_ALL;
+        !TAB && (sizeof(T) == 8 || TG <= 64) ? (TW_EARLY | TW_FINAL_POW) : TW_ALL;
     static constexpr int TW_PRE_C = (V & VAR_TW_C) ? tw_flip(TW_PRE_C0) : TW_PRE_C0;
     static constexpr bool OPS_EARLY_C = true;
     // pass A: FP64 loads its early-pass twiddles in one batch (1.3 % less
@@ -94,7 +108,8 @@ struct WaveCfg {
     // less time for the mixed ensemble than all in one batch, then 2.6 %
     // less than loading the final ones too)
     static constexpr int TW_PRE_A0 =
-        sizeof(T) == 8 ? (TW_EARLY | TW_FINAL_POW) : TG >= 128 ? TW_ALL : TW_FINAL_POW;
+        TAB ? TW_EARLY
+            : sizeof(T) == 8 ? (TW_EARLY | TW_FINAL_POW) : TG >= 128 ? TW_ALL : TW_FINAL_POW;
     static constexpr int TW_PRE_A = (V & VAR_TW_A) ? tw_flip(TW_PRE_A0) : TW_PRE_A0;
     // pass B: the lane's twiddles stay in registers for all of its row
     // transforms; FP64 has room next to the data (256 VGPRs) for the
@@ -104,22 +119,35 @@ struct WaveCfg {
     static constexpr int TW_PRE_B0 = sizeof(T) == 4 ? TW_ALL : (TW_EARLY | TW_FINAL_POW);
     static constexpr int TW_PRE_B = (V & VAR_TW_B) ? tw_flip(TW_PRE_B0) : TW_PRE_B0;
     // (one row per lane group: every twiddle in one batch by default)
-    static constexpr int TW_PRE_B1 = (V & VAR_TW_B) ? tw_flip(TW_ALL) : TW_ALL;
+    // (FP64 Np = 1152: powers, which fit three waves per SIMD, so that its
+    // 576 blocks run in one round: 22.9 -> 20.5 us)
+    static constexpr bool B3 = sizeof(T) == 8 && TG == 96;
+    static constexpr int TW_PRE_B10 = B3 ? (TW_EARLY | TW_FINAL_POW) : TW_ALL;
+    static constexpr int TW_PRE_B1 = (V & VAR_TW_B) ? tw_flip(TW_PRE_B10) : TW_PRE_B10;
     // pass B holds w and u + i v; a multi-wave group needs more registers
-    static constexpr int WPE_B = (sizeof(T) == 8 || TG > 64 || E == 24) ? 2 : 3;
-    static_assert(E * TG == NP && TG >= 2 && TG <= 256 && (TG & (TG - 1)) == 0,
+    static constexpr int WPE_B =
+        B3 || (!P2 && sizeof(T) == 4 && !PAIR_B) ? 3
+        : (sizeof(T) == 8 || TG > 64 || E == 24) ? 2 : 3;
+    static_assert(E * TG == NP && TG >= 2 && TG <= 256 &&
+                      (P2 || (E == 12 && TG % 3 == 0 && ((TG / 3) & (TG / 3 - 1)) == 0)),
                   "unsupported group FFT size");
+    static_assert(BLK % 64 == 0 && THR_B % 64 == 0, "blocks are whole waves");
 };
 
 // Tiles of passes A and B: LPB lines of NP elements (one lane group per
 // line, or per two rows in passB_pair).
-// The LDS slices are NP + 16 elements apart, so that the transposed reads
-// (LPB slices at one index) spread evenly over the banks.
+// The slices are spaced so that the transposed reads (LPB slices at one
+// index) spread evenly over the banks: NP + 16 elements apart for a power of
+// two; for 3*2^k PH / LPB past a multiple of the PH elements that cover the
+// 64 banks.
 template <typename T, int NP, int LPB, int V = 0>
 struct TileCfg {
     static constexpr int TG = WaveCfg<T, NP, V>::TG;
     static constexpr int BLK = LPB * TG;
-    static constexpr int SL = NP + 16;
+    static constexpr int PH = 256 / (int)sizeof(cpx<T>), SZ = LdsMap<TG>::size(NP);
+    static constexpr int SL = WaveCfg<T, NP, V>::P2
+                                  ? SZ + 16
+                                  : (SZ + PH - 1) / PH * PH + (LPB < PH ? PH / LPB : 1);
     static constexpr int LDS = LPB * SL;
     static_assert(LPB >= 1 && (LPB & (LPB - 1)) == 0 && BLK <= 1024, "bad tile");
 };
@@ -379,9 +407,9 @@ __device__ __forceinline__ void passA_body(int blk, int nblk, cpx<T> *lds,
     cpx<T> *slice = lds + g * SL;
     group_fft<T, E, TG, 1>(v, slice, t, gt);
     // transpose through LDS: the block's columns become LPB-element row segments
-    const int it = LdsPad<T>::idx(t);
+    const int it = LdsMap<TG>::idx(t);
 #pragma unroll
-    for (int s = 0; s < E; ++s) slice[LdsPad<T>::idx_sum(it, TG * s)] = v[s];
+    for (int s = 0; s < E; ++s) slice[LdsMap<TG>::idx_sum(it, TG * s)] = v[s];
     __syncthreads();
     // LPB * NP = E * BLK elements: element e = threadIdx.x + BLK m is row
     // e / LPB, column e % LPB of the tile (BLK = LPB * TG)
@@ -394,7 +422,7 @@ __device__ __forceinline__ void passA_body(int blk, int nblk, cpx<T> *lds,
 #pragma unroll
         for (int m = 0; m < E; ++m) {
             const int y = yb + TG * m;
-            col[(size_t)y * d.KG] = sl[LdsPad<T>::idx(y)];
+            col[(size_t)y * d.KG] = sl[LdsMap<TG>::idx(y)];
         }
     }
 }
@@ -459,7 +487,7 @@ __device__ __forceinline__ void passA_fused_body(int blk, int nblk, cpx<T> *lds,
         }
     });
     cpx<T> *slice = lds + g * SL;
-    const int it = LdsPad<T>::idx(t);
+    const int it = LdsMap<TG>::idx(t);
     const int gi = threadIdx.x % LPB, yb = threadIdx.x / LPB;
     // fields in the order w, u, v: w_hat first frees the column's registers
 #pragma unroll 1
@@ -476,7 +504,7 @@ __device__ __forceinline__ void passA_fused_body(int blk, int nblk, cpx<T> *lds,
         }
         group_fft<T, E, TG, 1>(v, slice, t, gt);
 #pragma unroll
-        for (int s = 0; s < E; ++s) slice[LdsPad<T>::idx_sum(it, TG * s)] = v[s];
+        for (int s = 0; s < E; ++s) slice[LdsMap<TG>::idx_sum(it, TG * s)] = v[s];
         __syncthreads();
         if (kx0 + gi < d.K) {
             cpx<T> *col = (f == 0 ? Gu : f == 1 ? Gv : Gw) + run * bt.sG + kx0 + gi;
@@ -484,7 +512,7 @@ __device__ __forceinline__ void passA_fused_body(int blk, int nblk, cpx<T> *lds,
 #pragma unroll
             for (int m = 0; m < E; ++m) {
                 const int y = yb + TG * m;
-                col[(size_t)y * d.KG] = sl[LdsPad<T>::idx(y)];
+                col[(size_t)y * d.KG] = sl[LdsMap<TG>::idx(y)];
             }
         }
         if (passA_tail(d.K, LPB) && kx0 + LPB == d.K - 1) { // block-uniform
@@ -631,9 +659,9 @@ __device__ __forceinline__ void passB_single(int blk, int nblk, cpx<T> *lds,
     for (int s = 0; s < E; ++s) v[s] = mk<T>(v[s].re * wr[s], v[s].im * wr[s]); // uw + i vw
     if (forward) {
         group_fft<T, E, TG, -1>(v, slice, t, gt);
-        const int it = LdsPad<T>::idx(t);
+        const int it = LdsMap<TG>::idx(t);
 #pragma unroll
-        for (int s = 0; s < E; ++s) slice[LdsPad<T>::idx_sum(it, TG * s)] = v[s];
+        for (int s = 0; s < E; ++s) slice[LdsMap<TG>::idx_sum(it, TG * s)] = v[s];
         __syncthreads();
         // k <= N/2 = NP/3 of the block's LPB rows, rows fastest: LPB-element
         // segments of the H columns
@@ -646,8 +674,8 @@ __device__ __forceinline__ void passB_single(int blk, int nblk, cpx<T> *lds,
             if (e < CNT) {
                 const int k = e / LPB, r = e % LPB;
                 const cpx<T> *sl = lds + r * SL;
-                const cpx<T> P = sl[LdsPad<T>::idx(k)];
-                cpx<T> Pc = sl[LdsPad<T>::idx((NP - k) % NP)];
+                const cpx<T> P = sl[LdsMap<TG>::idx(k)];
+                cpx<T> Pc = sl[LdsMap<TG>::idx((NP - k) % NP)];
                 Pc.im = -Pc.im;
                 const cpx<T> su = add(P, Pc), df = sub(P, Pc);
                 Huw[(size_t)k * NP + r] = mk<T>((T)0.5 * su.re, (T)0.5 * su.im);
@@ -745,9 +773,9 @@ __device__ __forceinline__ void passB_pair(int blk, int nblk, cpx<T> *lds,
 #pragma unroll
             for (int s = 0; s < E; ++s) x[s] = mk<T>(x[s].re * w[s], x[s].im * w[s]);
             group_fft<T, E, TG, -1>(x, sl, t, gt);
-            const int it = LdsPad<T>::idx(t);
+            const int it = LdsMap<TG>::idx(t);
 #pragma unroll
-            for (int s = 0; s < E; ++s) sl[LdsPad<T>::idx_sum(it, TG * s)] = x[s];
+            for (int s = 0; s < E; ++s) sl[LdsMap<TG>::idx_sum(it, TG * s)] = x[s];
         }
     };
     if constexpr (sizeof(T) != 4) load_uv(z, oa);
@@ -774,8 +802,8 @@ __device__ __forceinline__ void passB_pair(int blk, int nblk, cpx<T> *lds,
             if (e < CNT) {
                 const int k = e / LPB, r = e % LPB;
                 const cpx<T> *sl = lds + r * SL;
-                const cpx<T> P = sl[LdsPad<T>::idx(k)];
-                cpx<T> Pc = sl[LdsPad<T>::idx((NP - k) % NP)];
+                const cpx<T> P = sl[LdsMap<TG>::idx(k)];
+                cpx<T> Pc = sl[LdsMap<TG>::idx((NP - k) % NP)];
                 Pc.im = -Pc.im;
                 const cpx<T> su = add(P, Pc), df = sub(P, Pc);
                 Huw[(size_t)k * NP + r] = mk<T>((T)0.5 * su.re, (T)0.5 * su.im);
@@ -910,7 +938,7 @@ __device__ __forceinline__ void passC_finish(const cpx<T> (&v)[WaveCfg<T, NP, V>
     const T qx = (T)kx;
     const T inv_norm = (T)a.inv_norm; // multiplications instead of the
                                       // reference's divisions: <= 1 ulp
-    const int it = LdsPad<T>::idx(t);
+    const int it = LdsMap<TG>::idx(t);
     static_for<0, E / 2>([&](auto iI) {
         constexpr int i = decltype(iI)::value, s = 2 * i + HALF;
         if constexpr (pad_region<NP, TG, s>() != PAD_ZERO) {
@@ -920,7 +948,7 @@ __device__ __forceinline__ void passC_finish(const cpx<T> (&v)[WaveCfg<T, NP, V>
             // SetupTruncation's |k| <= kMax + 1e-10 (src/Spectral.F90:272-313)
             // is kx^2 + ky^2 <= (N/2)^2 on integer wavenumbers
             const bool keep = kx * kx + kyi * kyi <= H * H;
-            const cpx<T> o = other[LdsPad<T>::idx_sum(it, TG * s)]; // j = t + TG s
+            const cpx<T> o = other[LdsMap<TG>::idx_sum(it, TG * s)]; // j = t + TG s
             const cpx<T> Pr = HALF == 0 ? v[s] : o, Qr = HALF == 0 ? o : v[s];
             const cpx<T> P = mk<T>(Pr.re * inv_norm, Pr.im * inv_norm);
             const cpx<T> Q = mk<T>(Qr.re * inv_norm, Qr.im * inv_norm);
@@ -1010,10 +1038,10 @@ __device__ __forceinline__ void passC_half(int blk, cpx<T> *lds_all, int lane,
     group_fft<T, E, TG, -1>(v, mine, t, gt);
     if constexpr (!C::OPS_EARLY_C) op.load(t, Wn, Wst, Fc, col);
     // half 0 keeps the even s and hands over the odd s, half 1 the reverse
-    const int it = LdsPad<T>::idx(t);
+    const int it = LdsMap<TG>::idx(t);
 #pragma unroll
     for (int s = 0; s < E; ++s)
-        if ((s & 1) != HALF) mine[LdsPad<T>::idx_sum(it, TG * s)] = v[s];
+        if ((s & 1) != HALF) mine[LdsMap<TG>::idx_sum(it, TG * s)] = v[s];
     __syncthreads();
     // a run at its end time (dt = 0) stores nothing: its step-start state
     // stays in Wn (and Ws, which only this run's later stages read, is unused)

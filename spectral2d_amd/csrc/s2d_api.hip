@@ -771,14 +771,21 @@ int fused_steps_wave(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
 }
 
 // Padded sizes with compiled lane-group FFT kernels; 0 when the generic
-// kernels are used.
+// kernels are used (the runtime plans: other 2^a 3^b sizes). The compiled
+// kernels win wherever they exist. Measured per launch, generic / compiled,
+// FP64: Np = 144 pass A 8.2 / 4.9 us, B 35 / 6.5, C 8.2 / 5.4; Np = 1152
+// A 29 / 13, B 82 / 21, C 17 / 10 (the plans' index divisions, twiddle
+// loads in every pass and a barrier pair per radix; pass B's two rows per
+// lane group leave Np = 144 nine blocks of one wave).
 template <typename T>
 int wave_np(const s2d_ctx *c)
 {
     if (!c->wave_kernels) return 0;
     const int np = c->g.nxG;
     switch (np) {
-    case 96: case 192: case 384: case 768: case 1536: case 3072: return np;
+    case 96: case 192: case 384: case 768: case 1536: case 3072: // N = 2^k
+    case 144: case 288: case 576: case 1152: case 2304:          // N = 3 2^k
+        return np;
     }
     return 0;
 }
@@ -791,6 +798,11 @@ int wave_np(const s2d_ctx *c)
     case 768: { constexpr int NP = 768; CALL; } break;          \
     case 1536: { constexpr int NP = 1536; CALL; } break;        \
     case 3072: { constexpr int NP = 3072; CALL; } break;        \
+    case 144: { constexpr int NP = 144; CALL; } break;          \
+    case 288: { constexpr int NP = 288; CALL; } break;          \
+    case 576: { constexpr int NP = 576; CALL; } break;          \
+    case 1152: { constexpr int NP = 1152; CALL; } break;        \
+    case 2304: { constexpr int NP = 2304; CALL; } break;        \
     }
 
 template <typename T>
