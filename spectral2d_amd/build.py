@@ -15,7 +15,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libs2d.so")
 LIB_H5 = os.path.join(HERE, "libs2d_h5.so")
-SOURCES = [os.path.join(CSRC, "s2d_api.hip"), os.path.join(CSRC, "cnn.hip")]
+SOURCES = [os.path.join(CSRC, f) for f in ("s2d_api.hip", "ref_fft.hip", "cnn.hip")]
 ARCH = os.environ.get("S2D_OFFLOAD_ARCH", "gfx950")
 
 HIPCC_FLAGS = [

@@ -34,10 +34,12 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int TG>
+// BLK: the group's lanes span waves (or share them in another order than
+// TG consecutive lanes per group)
+template <int TG, bool BLK = (64 % TG != 0)>
 __device__ __forceinline__ void group_sync()
 {
-    if constexpr (64 % TG != 0)
+    if constexpr (BLK)
         __syncthreads();
     else
         wave_sync();
@@ -326,19 +328,19 @@ __device__ __forceinline__ void group_pass(cpx<T> (&v)[E], cpx<T> *lds, int t, c
     }
 }
 
-template <typename T, int E, int TG, int D, int Ls, class G>
+template <typename T, int E, int TG, int D, int Ls, bool BLK, class G>
 __device__ __forceinline__ void early_passes(cpx<T> (&v)[E], cpx<T> *lds, int t, const G &g)
 {
     if constexpr (Ls < TG) {
         constexpr int R = early_radix(E, TG / Ls);
         static_assert(E % R == 0 && (TG / Ls) % R == 0, "no early radix");
         group_pass<T, E, TG, R, Ls, D, G>(v, lds, t, g);
-        group_sync<TG>();
+        group_sync<TG, BLK>();
         const int it = LdsMap<TG>::idx(t);
 #pragma unroll
         for (int s = 0; s < E; ++s) v[s] = lds[LdsMap<TG>::idx_sum(it, TG * s)];
-        group_sync<TG>();
-        early_passes<T, E, TG, D, Ls * R, G>(v, lds, t, g);
+        group_sync<TG, BLK>();
+        early_passes<T, E, TG, D, Ls * R, BLK, G>(v, lds, t, g);
     }
 }
 
@@ -366,11 +368,11 @@ __device__ __forceinline__ void final_pass(cpx<T> (&v)[E], const G &g)
 // Full transform of the group: on entry v[s] = x[t + TG*s], on exit
 // v[s] = X[t + TG*s]. lds is the group's slice (LdsMap<TG>::size(n)); g holds
 // the lane's twiddles (GroupTw::load with the table of length n).
-template <typename T, int E, int TG, int D, int PRE>
+template <typename T, int E, int TG, int D, int PRE, bool BLK = (64 % TG != 0)>
 __device__ __forceinline__ void group_fft(cpx<T> (&v)[E], cpx<T> *lds, int t,
                                           const GroupTw<T, E, TG, PRE> &g)
 {
-    early_passes<T, E, TG, D, 1>(v, lds, t, g);
+    early_passes<T, E, TG, D, 1, BLK>(v, lds, t, g);
     final_pass<T, E, TG, D>(v, g);
 }
 

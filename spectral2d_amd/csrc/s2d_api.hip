@@ -25,6 +25,7 @@
 #include "kernels_ref.hpp"
 #include "kernels_spectrum.hpp"
 #include "kernels_closure.hpp"
+#include "ref_fft.hpp"
 #include "s2d_internal.hpp"
 
 using namespace s2d;
@@ -246,6 +247,30 @@ void launch(s2d_ctx *c, K kern, dim3 grid, dim3 block, size_t shmem, Args... arg
 
 // ----------------------------------------------- reference-layout FFTs
 
+// The compiled lane-group transforms (ref_fft.hip) serve the lengths they
+// have, 3 2^k and 9 2^k, which are those of padded grids; the runtime plans
+// below the others, powers of two among them: the unpadded grids of the
+// closure, whose network rounds its inputs to BF16 and turns another rounding
+// of an FP32 transform into a relative 5e-4 of the run. Measured per field of
+// 1536^2 FP64, plans / compiled: columns 38 / 14 us, rows 16 / 10 to 13.
+RefGrid ref_grid(const s2d_ctx *c)
+{
+    RefGrid g;
+    g.cI = c->g.cISize;
+    g.ny = c->g.nyG;
+    g.h = c->rowh.plan.n;
+    g.tw_col = c->col.tw;
+    g.tw_h = c->rowh.tw;
+    g.tw_x = c->tw_x;
+    g.norm = (double)c->g.nxG * (double)c->g.nyG;
+    g.x_mask = c->xMaskBool ? c->xMaskInd : -1;
+    g.y_mask = c->yMaskBool ? c->yMaskInd : -1;
+    g.kc2 = (long long)c->g.kxMU * c->g.kxMU; // SetupTruncation's |k| <= kMax + 1e-10
+    return g;
+}
+bool ref_col_on(const s2d_ctx *c) { return c->wave_kernels && ref_col_ok(c->g.nyG); }
+bool ref_row_on(const s2d_ctx *c) { return c->wave_kernels && ref_row_ok(c->rowh.plan.n); }
+
 // np planes ps elements apart (one by default)
 template <typename T, int E, int D>
 int launch_col_E(s2d_ctx *c, cpx<T> *data, int normalize, int np, long long ps)
@@ -270,6 +295,11 @@ int launch_col_E(s2d_ctx *c, cpx<T> *data, int normalize, int np, long long ps)
 template <typename T, int D>
 int launch_col(s2d_ctx *c, cpx<T> *data, int normalize, int np = 1, long long ps = 0)
 {
+    if (ref_col_on(c)) {
+        ref_col<T>(c->stream, ref_grid(c), data, D, normalize != 0, np, ps);
+        S2D_LAUNCHED(c, "k_ct_col");
+        return S2D_OK;
+    }
     switch (c->col.E) {
     case 12: return launch_col_E<T, 12, D>(c, data, normalize, np, ps);
     case 8: return launch_col_E<T, 8, D>(c, data, normalize, np, ps);
@@ -310,6 +340,11 @@ int launch_row_E(s2d_ctx *c, cpx<T> *data, int np, long long ps)
 template <typename T, bool R2C>
 int launch_row(s2d_ctx *c, cpx<T> *data, int np = 1, long long ps = 0)
 {
+    if (ref_row_on(c)) {
+        ref_row<T>(c->stream, ref_grid(c), data, R2C, np, ps);
+        S2D_LAUNCHED(c, "k_ct_row");
+        return S2D_OK;
+    }
     switch (c->rowh.E) {
     case 12: return launch_row_E<T, 12, R2C>(c, data, np, ps);
     case 8: return launch_row_E<T, 8, R2C>(c, data, np, ps);
@@ -416,9 +451,32 @@ int op_vorticity(s2d_ctx *c, int u, int v, int w)
     return S2D_OK;
 }
 
+// ComputeRHS (stage 0), or ComputeRHS and the RK stage's update with
+// ComputePsi and Truncate (stages 1, 2, 3; w is W, then WS), in three launches
+// (ref_fft.hpp). The slots then hold what the routines one by one leave in
+// them, except that stages 1 and 2 leave U, V and DW undefined.
+template <typename T>
+int op_rhs_fused(s2d_ctx *c, double nu, int u, int v, int w, int psi, int dW, int stage = 0,
+                 double dt = 0.0)
+{
+    ref_rhs<T>(c->stream, ref_grid(c), F<T>(c, psi), F<T>(c, u), F<T>(c, v), F<T>(c, w),
+               F<T>(c, dW), nu, stage, dt, F<T>(c, S2D_FIELD_W),
+               F<T>(c, stage == 3 ? S2D_FIELD_W : S2D_FIELD_WS),
+               F<T>(c, stage == 3 ? S2D_FIELD_PSI : S2D_FIELD_PSIS));
+    S2D_LAUNCHED(c, "ComputeRHS");
+    return S2D_OK;
+}
+
 template <typename T>
 int op_rhs(s2d_ctx *c, double nu, int u, int v, int w, int psi, int dW)
 {
+    // (one slot in two roles: the routines' order decides what it holds)
+    const int f[5] = {u, v, w, psi, dW};
+    bool distinct = true;
+    for (int a = 0; a < 5; ++a)
+        for (int b = 0; b < a; ++b) distinct = distinct && f[a] != f[b];
+    if (distinct && ref_col_on(c) && ref_row_on(c))
+        return op_rhs_fused<T>(c, nu, u, v, w, psi, dW);
     S2D_TRY(op_velocity<T>(c, u, v, psi, 0)); // Spectral.F90:424-425
     S2D_TRY(op_c2r<T>(c, u));                 // :433-435
     S2D_TRY(op_c2r<T>(c, v));
@@ -471,6 +529,14 @@ int op_integrate(s2d_ctx *c, double nu, double dt)
 {
     const int W = S2D_FIELD_W, PSI = S2D_FIELD_PSI, U = S2D_FIELD_U, V = S2D_FIELD_V;
     const int WS = S2D_FIELD_WS, PSIS = S2D_FIELD_PSIS, DW = S2D_FIELD_DW;
+    if (ref_col_on(c) && ref_row_on(c)) {
+        S2D_TRY(op_rhs_fused<T>(c, nu, U, V, W, PSI, DW, 1, dt));
+        S2D_TRY(op_rhs_fused<T>(c, nu, U, V, WS, PSIS, DW, 2, dt));
+        S2D_TRY(op_rhs_fused<T>(c, nu, U, V, WS, PSIS, DW, 3, dt));
+        hipLaunchKernelGGL(k_advance_time, dim3(1), dim3(64), 0, c->stream, c->d_sc, dt);
+        S2D_LAUNCHED(c, "k_advance_time");
+        return S2D_OK;
+    }
     S2D_TRY(op_fill<T>(c, WS)); // :147-149
     S2D_TRY(op_fill<T>(c, PSIS));
     S2D_TRY(op_fill<T>(c, DW));
