@@ -390,35 +390,27 @@ __global__ void k_unpack(const cpx<T> *__restrict__ Wc, cpx<T> *__restrict__ Wre
 
 // -------------------------------------------------------- diagnostics
 
-// Per-block FP64 partial sums over the reference-layout vorticity:
-// [tke, enstrophy, palinstrophy, max|w|, nonfinite count].
+// One mode's share of [tke, enstrophy, palinstrophy, max|w|, nonfinite count].
 template <typename T>
-__global__ void k_diag_partial(const cpx<T> *__restrict__ W, int cI, int ny,
-                               const int *__restrict__ kx, const int *__restrict__ ky,
-                               int kxMG, double *__restrict__ part)
+__device__ __forceinline__ void diag_mode(cpx<T> w, int kx, int ky, int kxMG, double (&a)[5])
+{
+    const double re = (double)w.re, im = (double)w.im;
+    if (!(re == re && im == im) || fabs(re) > 1.0e300 || fabs(im) > 1.0e300) a[4] += 1.0;
+    const double q = (double)kx * kx + (double)ky * ky;
+    const double wt = (kx == 0 || kx == kxMG) ? 0.5 : 1.0; // weight/2 folded
+    const double e = re * re + im * im;
+    if (q > 0.0) a[0] += wt * e / q;
+    a[1] += wt * e;
+    a[2] += wt * e * q;
+    const double m = sqrt(e);
+    a[3] = m > a[3] ? m : a[3];
+}
+
+// The block's five sums (and maximum) in a fixed tree, to part[0..4].
+__device__ __forceinline__ void diag_block(const double (&a)[5], double *__restrict__ part)
 {
     __shared__ double sh[5][256];
-    double a0 = 0, a1 = 0, a2 = 0, a3 = 0, a4 = 0;
-    S2D_GRID_LOOP(k, (size_t)cI * ny)
-    {
-        const int i = (int)(k % cI), j = (int)(k / cI);
-        const cpx<T> w = W[k];
-        const double re = (double)w.re, im = (double)w.im;
-        if (!(re == re && im == im) || fabs(re) > 1.0e300 || fabs(im) > 1.0e300) a4 += 1.0;
-        const double q = (double)kx[i] * kx[i] + (double)ky[j] * ky[j];
-        const double wt = (kx[i] == 0 || kx[i] == kxMG) ? 0.5 : 1.0; // weight/2 folded
-        const double e = re * re + im * im;
-        if (q > 0.0) a0 += wt * e / q;
-        a1 += wt * e;
-        a2 += wt * e * q;
-        const double m = sqrt(e);
-        a3 = m > a3 ? m : a3;
-    }
-    sh[0][threadIdx.x] = a0;
-    sh[1][threadIdx.x] = a1;
-    sh[2][threadIdx.x] = a2;
-    sh[3][threadIdx.x] = a3;
-    sh[4][threadIdx.x] = a4;
+    for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] = a[q];
     __syncthreads();
     for (int o = blockDim.x / 2; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) {
@@ -432,7 +424,68 @@ __global__ void k_diag_partial(const cpx<T> *__restrict__ W, int cI, int ny,
         __syncthreads();
     }
     if (threadIdx.x == 0)
-        for (int q = 0; q < 5; ++q) part[(size_t)blockIdx.x * 5 + q] = sh[q][0];
+        for (int q = 0; q < 5; ++q) part[q] = sh[q][0];
+}
+
+// Per-block FP64 partial sums over the reference-layout vorticity.
+template <typename T>
+__global__ void k_diag_partial(const cpx<T> *__restrict__ W, int cI, int ny,
+                               const int *__restrict__ kx, const int *__restrict__ ky,
+                               int kxMG, double *__restrict__ part)
+{
+    double a[5] = {0, 0, 0, 0, 0};
+    S2D_GRID_LOOP(k, (size_t)cI * ny)
+    {
+        const int i = (int)(k % cI), j = (int)(k / cI);
+        diag_mode(W[k], kx[i], ky[j], kxMG, a);
+    }
+    diag_block(a, part + (size_t)blockIdx.x * 5);
+}
+
+// The same sums for run blockIdx.y of a batch, from the compact state: the
+// threads walk the reference layout in k_diag_partial's order and take the
+// kept modes (the others would add zeros), so that a run's sums are bitwise
+// those of its unpacked field, without unpacking it. Bound by the strided
+// reads of the compact columns, from L2. 256 mixed runs: 0.3 ms for all of
+// them where an unpack, a reduction and a wait for each took 10 ms.
+template <typename T>
+__global__ void k_diag_runs(const cpx<T> *__restrict__ Wc, long long sW, FusedDims d,
+                            double *__restrict__ part)
+{
+    Wc += (size_t)blockIdx.y * sW;
+    double a[5] = {0, 0, 0, 0, 0};
+    const unsigned cI = (unsigned)d.cI, n = cI * (unsigned)d.Np;
+    for (unsigned k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const unsigned j = k / cI, i = k - j * cI;
+        const int c = compact_row((int)j, d);
+        if ((int)i >= d.K || c < 0) continue;
+        const int ky = (int)j <= d.Np / 2 ? (int)j : (int)j - d.Np;
+        diag_mode(Wc[(size_t)i * d.KP + c], (int)i, ky, d.Np / 2, a);
+    }
+    diag_block(a, part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 5);
+}
+
+// Run blockIdx.x's five values from its nb blocks' partials, in block order.
+static __global__ __launch_bounds__(256) void k_diag_sum(const double *__restrict__ part, int nb,
+                                                  double *__restrict__ out)
+{
+    __shared__ double sh[256 * 5];
+    part += (size_t)blockIdx.x * nb * 5;
+    const int q = threadIdx.x;
+    double s = 0.0;
+    for (int b0 = 0; b0 < nb; b0 += 256) {
+        const int m = nb - b0 < 256 ? nb - b0 : 256;
+        __syncthreads();
+        for (int k = threadIdx.x; k < 5 * m; k += 256) sh[k] = part[(size_t)b0 * 5 + k];
+        __syncthreads();
+        if (q < 5)
+            for (int b = 0; b < m; ++b) {
+                const double x = sh[b * 5 + q];
+                if (q == 3) s = x > s ? x : s;
+                else s += x;
+            }
+    }
+    if (q < 5) out[(size_t)blockIdx.x * 5 + q] = s;
 }
 
 } // namespace s2d

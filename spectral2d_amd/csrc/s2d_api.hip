@@ -960,37 +960,15 @@ void wrote(s2d_ctx *c, int f)
     if (f == S2D_FIELD_W) c->compact_stale = true;
 }
 
-// Diagnostics of the W slot (reference layout) with run r's time and step
-// count; the caller has brought the W slot up to date.
-int diag_of(s2d_ctx *c, int run, s2d_diag *out)
+// Blocks of the diagnostics' reductions (at most n_red).
+int diag_blocks(const s2d_ctx *c)
 {
-    const size_t n = nc_of(c);
-    int blocks = grid_blocks(n, 256);
-    if (blocks > c->n_red) blocks = c->n_red;
-    if (c->precision == S2D_FP64)
-        hipLaunchKernelGGL(k_diag_partial<double>, dim3(blocks), dim3(256), 0, c->stream,
-                           F<double>(c, S2D_FIELD_W), c->g.cISize, c->g.nyG, c->d_kx, c->d_ky,
-                           c->g.kxMG, c->d_red);
-    else
-        hipLaunchKernelGGL(k_diag_partial<float>, dim3(blocks), dim3(256), 0, c->stream,
-                           F<float>(c, S2D_FIELD_W), c->g.cISize, c->g.nyG, c->d_kx, c->d_ky,
-                           c->g.kxMG, c->d_red);
-    S2D_LAUNCHED(c, "k_diag_partial");
-    std::vector<double> part((size_t)blocks * 5);
-    S2D_HIP(c, hipMemcpyAsync(part.data(), c->d_red, part.size() * sizeof(double),
-                              hipMemcpyDeviceToHost, c->stream));
-    DevScalars sc;
-    S2D_HIP(c, hipMemcpyAsync(&sc, c->d_sc + run, sizeof(sc), hipMemcpyDeviceToHost, c->stream));
-    S2D_TRY(sync(c));
-    double a[5] = {0, 0, 0, 0, 0};
-    for (int b = 0; b < blocks; ++b)
-        for (int q = 0; q < 5; ++q) {
-            double x = part[(size_t)b * 5 + q];
-            if (q == 3)
-                a[q] = x > a[q] ? x : a[q];
-            else
-                a[q] += x;
-        }
+    return std::min(grid_blocks(nc_of(c), 256), c->n_red);
+}
+
+// The sums a[5] and a run's scalars as s2d_diagnostics returns them.
+int diag_result(s2d_ctx *c, const double *a, const DevScalars &sc, s2d_diag *out)
+{
     out->tke = a[0];
     out->enstrophy = a[1];
     out->palinstrophy = a[2];
@@ -1001,8 +979,55 @@ int diag_of(s2d_ctx *c, int run, s2d_diag *out)
     return S2D_OK;
 }
 
+// Diagnostics of the W slot (reference layout) with run r's time and step
+// count; the caller has brought the W slot up to date.
+int diag_of(s2d_ctx *c, int run, s2d_diag *out)
+{
+    const int blocks = diag_blocks(c);
+    if (c->precision == S2D_FP64)
+        hipLaunchKernelGGL(k_diag_partial<double>, dim3(blocks), dim3(256), 0, c->stream,
+                           F<double>(c, S2D_FIELD_W), c->g.cISize, c->g.nyG, c->d_kx, c->d_ky,
+                           c->g.kxMG, c->d_red);
+    else
+        hipLaunchKernelGGL(k_diag_partial<float>, dim3(blocks), dim3(256), 0, c->stream,
+                           F<float>(c, S2D_FIELD_W), c->g.cISize, c->g.nyG, c->d_kx, c->d_ky,
+                           c->g.kxMG, c->d_red);
+    S2D_LAUNCHED(c, "k_diag_partial");
+    double *sums = c->d_red + (size_t)blocks * 5;
+    hipLaunchKernelGGL(k_diag_sum, dim3(1), dim3(256), 0, c->stream, c->d_red, blocks, sums);
+    S2D_LAUNCHED(c, "k_diag_sum");
+    double a[5];
+    S2D_HIP(c, hipMemcpyAsync(a, sums, sizeof(a), hipMemcpyDeviceToHost, c->stream));
+    DevScalars sc;
+    S2D_HIP(c, hipMemcpyAsync(&sc, c->d_sc + run, sizeof(sc), hipMemcpyDeviceToHost, c->stream));
+    S2D_TRY(sync(c));
+    return diag_result(c, a, sc, out);
+}
+
+// The diagnostics' sums of every run of a batch from the compact state (5 per
+// run) and the runs' scalars, enqueued without a wait.
+template <typename T>
+int op_diag_runs(s2d_ctx *c, double *sums, DevScalars *sc)
+{
+    const int blocks = diag_blocks(c), M = c->nruns;
+    double *d_sums = c->d_red + (size_t)5 * M * blocks;
+    for (int r = 0; r < M; r += 32768) { // (runs on blockIdx.y)
+        hipLaunchKernelGGL(k_diag_runs<T>, dim3(blocks, std::min(M - r, 32768)), dim3(256), 0,
+                           c->stream, (const cpx<T> *)c->Wn + r * c->sW, c->sW, fdims(c),
+                           c->d_red + (size_t)5 * r * blocks);
+        S2D_LAUNCHED(c, "k_diag_runs");
+    }
+    hipLaunchKernelGGL(k_diag_sum, dim3(M), dim3(256), 0, c->stream, c->d_red, blocks, d_sums);
+    S2D_LAUNCHED(c, "k_diag_sum");
+    S2D_HIP(c, hipMemcpyAsync(sums, d_sums, sizeof(double) * 5 * M, hipMemcpyDeviceToHost,
+                              c->stream));
+    S2D_HIP(c, hipMemcpyAsync(sc, c->d_sc, sizeof(DevScalars) * M, hipMemcpyDeviceToHost,
+                              c->stream));
+    return S2D_OK;
+}
+
 // ComputeSpectrum of the PSI slot (brought up to date by the caller):
-// device shell sums, host mode counts and moments in shell order.
+// device shell sums and mode counts, host moments in shell order.
 // The shell spectrum of the psi slot fa (fb < 0), or of the velocity
 // spectra in slots fa (u) and fb (v).
 int spectrum_of(s2d_ctx *c, double nu, double *ek, int *cnt, double *tke, double *eps,
@@ -1010,54 +1035,24 @@ int spectrum_of(s2d_ctx *c, double nu, double *ek, int *cnt, double *tke, double
 {
     const s2d_grid &g = c->g;
     const int nb = s2d_spectrum_bins(&g);
-    // the reduction buffer holds 6 n_red doubles (>= 3072: every shell count
-    // up to N = 2048); larger grids take a buffer of their own
-    double *d_ek = c->d_red, *own = nullptr;
-    if ((size_t)nb > 6 * (size_t)c->n_red) {
-        S2D_HIP(c, hipMalloc((void **)&own, sizeof(double) * nb));
-        d_ek = own;
-    }
-    const int fv = fb < 0 ? fa : fb;
-    if (c->precision == S2D_FP64) {
-        if (fb < 0)
-            hipLaunchKernelGGL((k_spectrum<double, false>), dim3(nb), dim3(256), 0, c->stream,
-                               F<double>(c, fa), F<double>(c, fv), g.cISize, g.nyG, g.kxMG,
-                               g.kyMG, c->xMaskBool, c->yMaskBool, d_ek);
-        else
-            hipLaunchKernelGGL((k_spectrum<double, true>), dim3(nb), dim3(256), 0, c->stream,
-                               F<double>(c, fa), F<double>(c, fv), g.cISize, g.nyG, g.kxMG,
-                               g.kyMG, c->xMaskBool, c->yMaskBool, d_ek);
-    } else {
-        if (fb < 0)
-            hipLaunchKernelGGL((k_spectrum<float, false>), dim3(nb), dim3(256), 0, c->stream,
-                               F<float>(c, fa), F<float>(c, fv), g.cISize, g.nyG, g.kxMG,
-                               g.kyMG, c->xMaskBool, c->yMaskBool, d_ek);
-        else
-            hipLaunchKernelGGL((k_spectrum<float, true>), dim3(nb), dim3(256), 0, c->stream,
-                               F<float>(c, fa), F<float>(c, fv), g.cISize, g.nyG, g.kxMG,
-                               g.kyMG, c->xMaskBool, c->yMaskBool, d_ek);
-    }
-    const hipError_t el = hipGetLastError();
-    std::vector<double> h((size_t)nb);
-    const hipError_t ec =
-        hipMemcpyAsync(h.data(), d_ek, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream);
-    const hipError_t es = hipStreamSynchronize(c->stream);
-    if (own) (void)hipFree(own);
-    if (el != hipSuccess) return fail(c, S2D_ERR_HIP, "launch of k_spectrum failed");
-    if (ec != hipSuccess || es != hipSuccess)
-        return fail(c, S2D_ERR_HIP, "read-back of the spectrum failed");
-    // mode counts of the padded spectrum, weights 1 / 2 (src/Analysis.F90:389-395)
-    if (cnt) {
-        for (int b = 0; b < nb; ++b) cnt[b] = 0;
-        for (int j = 0; j < g.nyG; ++j)
-            for (int i = 0; i < g.cISize; ++i) {
-                const long long m = (long long)c->kx[i] * c->kx[i] + (long long)c->ky[j] * c->ky[j];
-                long long b = (long long)std::sqrt((double)m);
-                while (b * b > m) --b;
-                if (m > b * b + b) ++b; // floor(sqrt(m) + 1/2)
-                cnt[b] += (c->kx[i] == 0 || c->kx[i] == g.kxMG) ? 1 : 2;
-            }
-    }
+    double *d_ek = c->d_red; // nb sums, then nb counts
+    int *d_cnt = reinterpret_cast<int *>(d_ek + nb);
+    auto shells = [&](auto uv, auto zero) {
+        using T = decltype(zero);
+        hipLaunchKernelGGL((k_spectrum<T, decltype(uv)::value>), dim3(nb), dim3(256), 0, c->stream,
+                           F<T>(c, fa), F<T>(c, fb < 0 ? fa : fb), g.cISize, g.nyG, g.kxMG,
+                           g.kyMG, c->xMaskBool, c->yMaskBool, d_ek, d_cnt);
+    };
+    if (c->precision == S2D_FP64)
+        fb < 0 ? shells(std::false_type{}, 0.0) : shells(std::true_type{}, 0.0);
+    else
+        fb < 0 ? shells(std::false_type{}, 0.0f) : shells(std::true_type{}, 0.0f);
+    S2D_LAUNCHED(c, "k_spectrum");
+    std::vector<double> h((size_t)nb + (nb + 1) / 2);
+    S2D_HIP(c, hipMemcpyAsync(h.data(), d_ek, (sizeof(double) + sizeof(int)) * nb,
+                              hipMemcpyDeviceToHost, c->stream));
+    S2D_TRY(sync(c));
+    if (cnt) std::memcpy(cnt, h.data() + nb, sizeof(int) * nb);
     double t = 0.0, e = 0.0, z = 0.0; // src/Analysis.F90:439-448 (dk = 1)
     for (int b = 0; b < nb; ++b) {
         const double kb = (double)b;
@@ -1522,7 +1517,10 @@ int create_ctx(int nx, int ny, int dealias, int precision, int nruns, hipStream_
         return bail(S2D_ERR_UNSUPPORTED);
     }
     c->n_red = 512 > nruns ? 512 : nruns;
-    if (hipMalloc(&c->d_red, sizeof(double) * 6 * c->n_red)) {
+    // the diagnostics' partials and sums of every run, a spectrum's shells
+    const size_t nred = std::max((size_t)5 * nruns * (diag_blocks(c) + 1),
+                                 2 * (size_t)s2d_spectrum_bins(&c->g));
+    if (hipMalloc(&c->d_red, sizeof(double) * std::max(nred, 6 * (size_t)c->n_red))) {
         c->err = "device allocation of reduction buffers failed";
         return bail(S2D_ERR_ALLOC);
     }
