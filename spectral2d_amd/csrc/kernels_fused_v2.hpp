@@ -67,13 +67,18 @@ struct WaveCfg {
     // sizes is what bounds their neighbours: latency (one round of blocks) up
     // to Np = 1152, the 256 MB cache and VALU issue at 2304. FP64 Np = 1152:
     // 13, 21 and 10 us for A, B and C (26, 35 and 28 MB of algorithmic traffic)
+    // powers of two: 256 lanes a block; up to Np = 384, where that makes 3 to
+    // 48 blocks, one wave, which spreads a launch over more CUs (pass B FP64
+    // Np = 96 / 192 / 384: 8.0 / 8.4 / 9.5 -> 5.4 / 5.6 / 7.1 us, pass A 5.8 /
+    // 5.4 / 6.0 -> 4.7 / 4.8 / 5.2; at 768 two waves are 4 % slower than four)
+    static constexpr int THR_P2 = NP <= 384 ? 64 : 256;
     static constexpr int THR3_A = sizeof(T) == 4 && TG > 12 ? 384 : 192;
     static constexpr int LPB_A = !P2 ? (TG >= 192 ? 2 : THR3_A / TG)
-                                 : TG >= 256 ? (sizeof(T) == 4 ? 2 : 1) : 256 / TG;
+                                 : TG >= 256 ? (sizeof(T) == 4 ? 2 : 1) : THR_P2 / TG;
     // pass B: two rows per lane group from Np = 1536 up (passB_pair)
     static constexpr bool PAIR_B = (NP >= 1536) != ((V & VAR_PAIR) != 0);
     static constexpr int LPB_B = PAIR_B ? 2 : !P2 ? 192 / TG
-                                 : TG >= 128 && sizeof(T) == 8 ? 1 : TG >= 256 ? 2 : 256 / TG;
+                                 : TG >= 128 && sizeof(T) == 8 ? 1 : TG >= 256 ? 2 : THR_P2 / TG;
     static constexpr int THR_B = PAIR_B ? LPB_B * TG / 2 : LPB_B * TG; // lanes per block
     // pass C: column groups per half, two halves per block (whole waves each)
     static constexpr int GPB = !P2 ? 192 / TG : TG >= 64 ? 1 : 64 / TG;
