@@ -122,11 +122,44 @@ __device__ __forceinline__ uint32_t pk_bf16(float lo, float hi)
     return __builtin_bit_cast(uint32_t, v);
 }
 
+__device__ __forceinline__ uint4 pk_bf16x8(const float (&v)[8])
+{
+    return uint4{pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3]), pk_bf16(v[4], v[5]),
+                 pk_bf16(v[6], v[7])};
+}
+// The eight BF16 values of a 16-byte chunk.
+__device__ __forceinline__ void unpack_bf16x8(uint4 u, float (&v)[8])
+{
+    const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        v[2 * k] = bf2f((u16)(w[k] & 0xffffu));
+        v[2 * k + 1] = bf2f((u16)(w[k] >> 16));
+    }
+}
+
 // LDS rows of 64 BF16 channels (eight 16-byte chunks): chunk c of row r is
 // stored at chunk c ^ (r & 7) of the row, so that any eight consecutive rows
 // an operand read takes (eight lanes, one chunk each) fall on distinct banks
 // (measured: 3 % less time than c ^ ((r >> 1) & 7), which spreads sixteen).
 __device__ __forceinline__ int sw_chunk(int r, int c) { return r * 8 + (c ^ (r & 7)); }
+
+// Channel of row r (0..15) of MFMA output tile mt (0..3): a lane, which holds
+// rows 4 g .. 4 g + 3 of every tile, then has the eight consecutive channels
+// 32 h + 8 g .. + 7 in tiles 2 h and 2 h + 1 and stores them as 16 bytes; the
+// four lanes of a pixel cover 64 bytes per store. (With channel 16 mt + r each
+// store was 8 bytes, 32 per pixel: twice the store instructions and lines
+// touched; k_conv64 forward 117 -> 112 us, without z 100 -> 92, backward data
+// 121 -> 116, k_conv_in 99 -> 79 at 256^2 x 16, the same bits.)
+__host__ __device__ constexpr int co_of(int mt, int r)
+{
+    return 32 * (mt >> 1) + 8 * (r >> 2) + 4 * (mt & 1) + (r & 3);
+}
+// its inverse: 16 mt + r of channel co
+__host__ __device__ constexpr int row_of_co(int co)
+{
+    return 16 * (2 * (co >> 5) + ((co >> 2) & 1)) + 4 * ((co >> 3) & 3) + (co & 3);
+}
 
 // ------------------------------------------------------------ layer 0
 // z0[p][co] = b0[co] + sum_t sum_ci W0[t][ci][co] xs_ci[p + off_t], on the
@@ -156,7 +189,7 @@ __global__ __launch_bounds__(256) void k_conv_in(const float *__restrict__ x0,
         const long long o = n * sN + (long long)y2 * ld + x2;
         xs[r][j] = pk_bf16(s0 * x0[o], s1 * x1[o]);
     }
-    // A: lane (co = 16 mt + l16, k = 8 g4 + e): W0[t][ci][co] for k = 2 t + ci < 18
+    // A: lane (co = co_of(mt, l16), k = 8 g4 + e): W0[t][ci][co] for k = 2 t + ci < 18
     bf16x8_t av[4];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
@@ -164,7 +197,7 @@ __global__ __launch_bounds__(256) void k_conv_in(const float *__restrict__ x0,
 #pragma unroll
         for (int e2 = 0; e2 < 4; ++e2) {
             const int k = 8 * g4 + 2 * e2; // k and k + 1: tap k / 2, ci 0 and 1
-            const int co = 16 * mt + l16;
+            const int co = co_of(mt, l16);
             w[e2] = k < 18 ? pk_bf16(P[OFF_W0 + (k / 2 * 2 + 0) * CH + co],
                                      P[OFF_W0 + (k / 2 * 2 + 1) * CH + co])
                            : 0u;
@@ -176,7 +209,7 @@ __global__ __launch_bounds__(256) void k_conv_in(const float *__restrict__ x0,
     float4 bb[4];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
-        bb[mt] = *reinterpret_cast<const float4 *>(P + OFF_B0 + 16 * mt + 4 * g4);
+        bb[mt] = *reinterpret_cast<const float4 *>(P + OFF_B0 + co_of(mt, 4 * g4));
     __syncthreads();
     // B: lane (pixel 32 w + 16 nt + l16, k = 8 g4 + e): the pair of tap (8 g4 + e) / 2
     float4_t acc[4][2];
@@ -195,18 +228,26 @@ __global__ __launch_bounds__(256) void k_conv_in(const float *__restrict__ x0,
             acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 av[mt], bv, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
     }
-    // lane: channels co = 16 mt + 4 g4 + i of pixel xb + 32 w + 16 nt + l16
+    // lane: channels 32 h + 8 g4 .. + 7 (tiles 2 h, 2 h + 1) of pixel xb + 32 w + 16 nt + l16
 #pragma unroll
     for (int nt = 0; nt < 2; ++nt) {
-        const size_t pix = ((size_t)row * W + xb + 32 * wv + 16 * nt + l16) * CH + 4 * g4;
+        const size_t pix = ((size_t)row * W + xb + 32 * wv + 16 * nt + l16) * CH + 8 * g4;
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            const float v[4] = {acc[mt][nt][0] + bb[mt].x, acc[mt][nt][1] + bb[mt].y,
-                                acc[mt][nt][2] + bb[mt].z, acc[mt][nt][3] + bb[mt].w};
-            const size_t o = pix + 16 * mt;
-            if (z) *reinterpret_cast<uint2 *>(z + o) = uint2{pk_bf16(v[0], v[1]), pk_bf16(v[2], v[3])};
-            *reinterpret_cast<uint2 *>(a + o) =
-                uint2{pk_bf16(gelu(v[0]), gelu(v[1])), pk_bf16(gelu(v[2]), gelu(v[3]))};
+        for (int h = 0; h < 2; ++h) {
+            float v[8];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int mt = 2 * h + m;
+                v[4 * m + 0] = acc[mt][nt][0] + bb[mt].x;
+                v[4 * m + 1] = acc[mt][nt][1] + bb[mt].y;
+                v[4 * m + 2] = acc[mt][nt][2] + bb[mt].z;
+                v[4 * m + 3] = acc[mt][nt][3] + bb[mt].w;
+            }
+            const size_t o = pix + 32 * h;
+            if (z) *reinterpret_cast<uint4 *>(z + o) = pk_bf16x8(v);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = gelu(v[k]);
+            *reinterpret_cast<uint4 *>(a + o) = pk_bf16x8(v);
         }
     }
 }
@@ -224,8 +265,9 @@ __global__ __launch_bounds__(256) void k_conv_in(const float *__restrict__ x0,
 //           gelu(acc + bias) -> ao (BF16)
 //   mode 1: out = acc * gelu'(zp) -> zo (BF16)   (the backward data pass:
 //           in = dZ_l, wt = the flipped transpose of W_l, zp = z_{l-1})
-// wt: BF16 [9][64 co][64 ci]. Output stores: each lane writes four
-// channels (8 bytes) of one pixel per tile.
+// wt: BF16 [9][64 co][64 ci]; in LDS the rows of a tap are in tile order
+// (row_of_co). Output stores: each lane writes eight channels (16 bytes) of
+// one pixel per two tiles.
 constexpr int CV_SEG = 64, CV_PX = CV_SEG + 2, CV_RING = 10, CV_THREADS = 512;
 constexpr int CV_ROWCH = CV_PX * 8; // 16-byte chunks of a ring row
 
@@ -263,7 +305,8 @@ __global__ __launch_bounds__(CV_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 #pragma unroll
         for (int k = 0; k < NWC; ++k) {
             const int q = tid + CV_THREADS * k;
-            sw[sw_chunk(q >> 3, q & 7)] = vw[k];
+            const int r = q >> 3; // tap * 64 + co
+            sw[sw_chunk((r & ~(CH - 1)) + row_of_co(r & (CH - 1)), q & 7)] = vw[k];
         }
 #pragma unroll
         for (int k = 0; k < NRC; ++k) {
@@ -350,44 +393,48 @@ __global__ __launch_bounds__(CV_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
             __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);                          // MFMAs
         });
     };
-    // lane: channels co = 16 mt + 4 g4 + i of pixel x0 + 16 nt + l16 of image row y.
+    // lane: channels 32 h + 8 g4 .. + 7 (tiles 2 h, 2 h + 1) of pixel
+    // x0 + 16 nt + l16 of image row y.
     // No global load follows a store here: vmcnt counts both, so a load
     // issued after the stores would wait for all of them (measured: 24 %
     // of the forward time, with a bias load per tile). The bias comes from
-    // LDS; the backward pass loads its 16 z values before the first store.
+    // LDS; the backward pass loads its 8 chunks of z before the first store.
     auto epilogue = [&](int y) __attribute__((always_inline)) {
-        const size_t pix0 = (((size_t)n * H + y) * W + x0 + l16) * CH + 4 * g4;
+        const size_t pix0 = (((size_t)n * H + y) * W + x0 + l16) * CH + 8 * g4;
         if (mode == 0) {
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt) {
+            for (int q = 0; q < 8; ++q) { // nt = q / 2, h = q % 2
+                const int nt = q >> 1, h = q & 1;
+                const size_t o = pix0 + (size_t)16 * nt * CH + 32 * h;
+                float v[8];
 #pragma unroll
-                for (int mt = 0; mt < 4; ++mt) {
-                    const size_t o = pix0 + (size_t)16 * nt * CH + 16 * mt;
-                    const float4 bb = *reinterpret_cast<const float4 *>(sb + 16 * mt + 4 * g4);
-                    const float v0 = acc[mt][nt][0] + bb.x, v1 = acc[mt][nt][1] + bb.y,
-                                v2 = acc[mt][nt][2] + bb.z, v3 = acc[mt][nt][3] + bb.w;
-                    if (zo)
-                        *reinterpret_cast<uint2 *>(zo + o) = uint2{pk_bf16(v0, v1), pk_bf16(v2, v3)};
-                    *reinterpret_cast<uint2 *>(ao + o) =
-                        uint2{pk_bf16(gelu(v0), gelu(v1)), pk_bf16(gelu(v2), gelu(v3))};
+                for (int m = 0; m < 2; ++m) {
+                    const float4 bb =
+                        *reinterpret_cast<const float4 *>(sb + 32 * h + 8 * g4 + 4 * m);
+                    const float4_t a = acc[2 * h + m][nt];
+                    v[4 * m + 0] = a[0] + bb.x, v[4 * m + 1] = a[1] + bb.y;
+                    v[4 * m + 2] = a[2] + bb.z, v[4 * m + 3] = a[3] + bb.w;
                 }
+                if (zo) *reinterpret_cast<uint4 *>(zo + o) = pk_bf16x8(v);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = gelu(v[k]);
+                *reinterpret_cast<uint4 *>(ao + o) = pk_bf16x8(v);
             }
         } else {
-            uint2 zz[16]; // tile q: nt = q / 4, mt = q % 4
+            uint4 zz[8];
 #pragma unroll
-            for (int q = 0; q < 16; ++q)
-                zz[q] = *reinterpret_cast<const uint2 *>(zp + pix0 + (size_t)16 * (q >> 2) * CH +
-                                                         16 * (q & 3));
+            for (int q = 0; q < 8; ++q)
+                zz[q] = *reinterpret_cast<const uint4 *>(zp + pix0 + (size_t)16 * (q >> 1) * CH +
+                                                         32 * (q & 1));
 #pragma unroll
-            for (int q = 0; q < 16; ++q) {
-                const int nt = q >> 2, mt = q & 3;
-                const float4_t a = acc[mt][nt];
-                const float g0 = a[0] * gelu_grad(bf2f((u16)(zz[q].x & 0xffffu)));
-                const float g1 = a[1] * gelu_grad(bf2f((u16)(zz[q].x >> 16)));
-                const float g2 = a[2] * gelu_grad(bf2f((u16)(zz[q].y & 0xffffu)));
-                const float g3 = a[3] * gelu_grad(bf2f((u16)(zz[q].y >> 16)));
-                *reinterpret_cast<uint2 *>(zo + pix0 + (size_t)16 * nt * CH + 16 * mt) =
-                    uint2{pk_bf16(g0, g1), pk_bf16(g2, g3)};
+            for (int q = 0; q < 8; ++q) {
+                const int nt = q >> 1, h = q & 1;
+                float v[8];
+                unpack_bf16x8(zz[q], v);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v[k] = acc[2 * h + (k >> 2)][nt][k & 3] * gelu_grad(v[k]);
+                *reinterpret_cast<uint4 *>(zo + pix0 + (size_t)16 * nt * CH + 32 * h) =
+                    pk_bf16x8(v);
             }
         }
     };
@@ -566,44 +613,67 @@ __global__ __launch_bounds__(DW_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 // ------------------------------------------------------------ layer 5
 // y[p] = b5 + sum_t sum_ci W5[t][ci] a[p + off_t][ci]  (FP32 output, dense
 // [B][H][W]).
-// Grid (W / 32, B * H): 8 lanes per pixel, 8 channels each.
+// Grid (W / 32, B * H / CO_ROWS): 8 lanes per pixel, 8 channels each, CO_ROWS
+// rows of a column per lane: an input chunk is loaded and unpacked once for
+// the three output rows it enters (one row per lane loaded and unpacked every
+// chunk three times over: 66 us against 56 at 256^2 x 16, 27 by HBM). Every
+// output keeps its order of additions: taps, then channels, then lanes.
+constexpr int CO_ROWS = 4;
 __global__ __launch_bounds__(256) void k_conv_out(const u16 *__restrict__ a,
                                                   const float *__restrict__ P,
                                                   float *__restrict__ y, int B, int H, int W)
 {
     constexpr int NW = 9 * CH + 1, NWI = (NW + 255) / 256;
-    __shared__ float w[NW];
-    const int row = blockIdx.y, n = row / H, yy = row - n * H; // uniform
+    __shared__ __align__(16) float w[NW];
+    const int row = blockIdx.y * CO_ROWS, n = row / H, yy = row - n * H; // uniform (CO_ROWS | H)
     const int xx = blockIdx.x * 32 + (threadIdx.x >> 3), c8 = 8 * (threadIdx.x & 7);
-    // every load first (weights and the nine input chunks), then the arithmetic
+    // every load first (weights and the input chunks), then the arithmetic
     float wv[NWI];
-    uint4 v[9];
+    uint4 v[CO_ROWS + 2][3];
 #pragma unroll
     for (int i = 0; i < NWI; ++i) {
         const int j = threadIdx.x + 256 * i;
         if (j < NW) wv[i] = P[OFF_W5 + j]; // OFF_B5 = OFF_W5 + 9 CH
     }
 #pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        const int y2 = wrap(yy + t / 3 - 1, H), x2 = wrap(xx + t % 3 - 1, W);
-        v[t] = *reinterpret_cast<const uint4 *>(a + (((size_t)n * H + y2) * W + x2) * CH + c8);
-    }
+    for (int r = 0; r < CO_ROWS + 2; ++r)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+            const int y2 = wrap(yy + r - 1, H), x2 = wrap(xx + dx - 1, W);
+            v[r][dx] =
+                *reinterpret_cast<const uint4 *>(a + (((size_t)n * H + y2) * W + x2) * CH + c8);
+        }
 #pragma unroll
     for (int i = 0; i < NWI; ++i) {
         const int j = threadIdx.x + 256 * i;
         if (j < NW) w[j] = j < 9 * CH ? bfr(wv[i]) : wv[i];
     }
     __syncthreads();
-    float s = 0.f;
+    float s[CO_ROWS];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        const u16 *h = reinterpret_cast<const u16 *>(&v[t]);
-        for (int k = 0; k < 8; ++k) s += bf2f(h[k]) * w[t * CH + c8 + k];
+    for (int o = 0; o < CO_ROWS; ++o) s[o] = 0.f;
+#pragma unroll
+    for (int r = 0; r < CO_ROWS + 2; ++r)
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+            float f[8];
+            unpack_bf16x8(v[r][dx], f);
+#pragma unroll
+            for (int dy = 0; dy < 3; ++dy) { // input row yy + r - 1 = output row yy + o, tap row dy
+                const int o = r - dy;
+                if (o < 0 || o >= CO_ROWS) continue;
+                const float *wt = w + (3 * dy + dx) * CH + c8;
+#pragma unroll
+                for (int k = 0; k < 8; ++k) s[o] += f[k] * wt[k];
+            }
+        }
+#pragma unroll
+    for (int o = 0; o < CO_ROWS; ++o) {
+        s[o] += __shfl_xor(s[o], 1);
+        s[o] += __shfl_xor(s[o], 2);
+        s[o] += __shfl_xor(s[o], 4);
+        if ((threadIdx.x & 7) == 0) y[(size_t)(row + o) * W + xx] = s[o] + w[9 * CH];
     }
-    s += __shfl_xor(s, 1);
-    s += __shfl_xor(s, 2);
-    s += __shfl_xor(s, 4);
-    if ((threadIdx.x & 7) == 0) y[(size_t)row * W + xx] = s + w[9 * CH];
 }
 
 // Scaled output planes: out[n][yy][xx] (row pitch ld, sample stride sN) =
@@ -648,11 +718,14 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ y,
 }
 
 // Backward of layer 5: dZ4[q][ci] = (sum_t dy[q - off_t] W5[t][ci]) *
-// gelu'(z4[q][ci]) (BF16). Eight lanes per pixel, eight channels each; a
-// block takes OB_PX pixels, OB_PPT per lane, whose loads are all issued
-// before the first store (a loop with a store between loads waits for the
-// store at every load: vmcnt counts both). The rounded W5 sits in LDS.
-constexpr int OB_PPT = 4, OB_PX = 256 / 8 * OB_PPT;
+// gelu'(z4[q][ci]) (BF16). Eight lanes per pixel, eight channels each,
+// OB_ROWS rows of a column per lane (their dy window shared), whose loads are
+// all issued before the first store (a loop with a store between loads waits
+// for the store at every load: vmcnt counts both). The rounded W5 sits in LDS.
+// Bound by VALU issue (nine multiply-adds and a gelu' per value): 97 us with a
+// window of its own for every pixel, 83 so, at 256^2 x 16; 53 by HBM.
+// Grid (W / 32, B * H / OB_ROWS).
+constexpr int OB_ROWS = 4;
 __global__ __launch_bounds__(256) void k_out_bwd_data(const float *__restrict__ dy,
                                                       const float *__restrict__ P,
                                                       const u16 *__restrict__ z4,
@@ -660,22 +733,19 @@ __global__ __launch_bounds__(256) void k_out_bwd_data(const float *__restrict__ 
 {
     __shared__ __align__(16) float ws[9 * CH];
     for (int i = threadIdx.x; i < 9 * CH; i += 256) ws[i] = bfr(P[OFF_W5 + i]);
-    const int c8 = 8 * (threadIdx.x & 7), npx = B * H * W; // pixels < 2^31 (s2d_cnn_create)
-    int qs[OB_PPT];
-    uint4 zz[OB_PPT];
-    float d[OB_PPT][9];
+    const int row = blockIdx.y * OB_ROWS, n = row / H, yy = row - n * H; // uniform (OB_ROWS | H)
+    const int xx = blockIdx.x * 32 + (threadIdx.x >> 3), c8 = 8 * (threadIdx.x & 7);
+    const size_t q0 = ((size_t)row * W + xx) * CH + c8;
+    uint4 zz[OB_ROWS];
+    float d[OB_ROWS + 2][3]; // dy at row yy - 1 + j, column xx - 1 + i
 #pragma unroll
-    for (int j = 0; j < OB_PPT; ++j) {
-        qs[j] = blockIdx.x * OB_PX + 32 * j + (int)(threadIdx.x >> 3);
-        const int q = qs[j] < npx ? qs[j] : npx - 1; // (past the end: loaded, not stored)
-        const int xx = q % W, yy = (q / W) % H, n = q / (W * H);
-        zz[j] = *reinterpret_cast<const uint4 *>(z4 + (size_t)q * CH + c8);
+    for (int j = 0; j < OB_ROWS; ++j)
+        zz[j] = *reinterpret_cast<const uint4 *>(z4 + q0 + (size_t)j * W * CH);
 #pragma unroll
-        for (int t = 0; t < 9; ++t) {
-            const int y2 = wrap(yy - (t / 3 - 1), H), x2 = wrap(xx - (t % 3 - 1), W);
-            d[j][t] = dy[((size_t)n * H + y2) * W + x2];
-        }
-    }
+    for (int j = 0; j < OB_ROWS + 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            d[j][i] = dy[((size_t)n * H + wrap(yy - 1 + j, H)) * W + wrap(xx - 1 + i, W)];
     __syncthreads();
     float w[9][8];
 #pragma unroll
@@ -686,28 +756,29 @@ __global__ __launch_bounds__(256) void k_out_bwd_data(const float *__restrict__ 
         w[t][4] = hi.x, w[t][5] = hi.y, w[t][6] = hi.z, w[t][7] = hi.w;
     }
 #pragma unroll
-    for (int j = 0; j < OB_PPT; ++j) {
-        const uint32_t zw[4] = {zz[j].x, zz[j].y, zz[j].z, zz[j].w};
-        float o[8];
+    for (int j = 0; j < OB_ROWS; ++j) {
+        float z[8], o[8];
+        unpack_bf16x8(zz[j], z);
 #pragma unroll
         for (int k = 0; k < 8; ++k) {
             float s = 0.f;
 #pragma unroll
-            for (int t = 0; t < 9; ++t) s += d[j][t] * w[t][k];
-            const u16 zh = (u16)((k & 1) ? zw[k >> 1] >> 16 : zw[k >> 1] & 0xffffu);
-            o[k] = s * gelu_grad(bf2f(zh));
+            for (int t = 0; t < 9; ++t) s += d[j + 2 - t / 3][2 - t % 3] * w[t][k]; // q - off_t
+            o[k] = s * gelu_grad(z[k]);
         }
-        if (qs[j] < npx)
-            *reinterpret_cast<uint4 *>(dz + (size_t)qs[j] * CH + c8) =
-                uint4{pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3]), pk_bf16(o[4], o[5]),
-                      pk_bf16(o[6], o[7])};
+        *reinterpret_cast<uint4 *>(dz + q0 + (size_t)j * W * CH) = pk_bf16x8(o);
     }
 }
 
 // Weight gradients of the thin layers: one block per 64-pixel column
-// segment of R rows of one sample; thread (channel = lane, pixel group =
-// wave) walks 16 pixels of each row, accumulates in FP32, and the four
-// waves' sums are added in LDS. Per-block partial sums, reduced by k_reduce.
+// segment of R rows of one sample. A lane takes eight channels (16 bytes) of
+// a column of pixels, eight lanes a pixel, and walks down the rows of the
+// segment's two 32-pixel halves: every activation is loaded once, its nine
+// neighbours of the one-channel side slide down with it. FP32 sums per lane;
+// the 32 columns' are added by shuffles, then over the four waves in LDS.
+// Per-block partial sums, reduced by k_reduce. (A lane per channel, 2-byte
+// loads, three rows of neighbours each: layer 5 87 us against 45, layer 0 84
+// against 60 at 256^2 x 16; 27 us each by HBM.)
 // R: GR, doubled (dividing H) while at least `width` blocks remain.
 constexpr int GR = 8, GSEG = 64, CNN_THIN_WIDTH = 512;
 int thin_rows(int B, int H, int W, int width)
@@ -721,8 +792,17 @@ int thin_blocks(int B, int H, int W, int width)
     return B * (H / thin_rows(B, H, W, width)) * (W / GSEG);
 }
 
-// Layer 5: dW5[t][ci] = sum_p dy[p] a4[p + off_t][ci], db5 = sum_p dy[p];
-// partial layout [t][ci] then db5.
+// The sum over a wave's eight pixel columns (lanes with the same lane & 7).
+__device__ __forceinline__ float add_columns(float v)
+{
+    v += __shfl_xor(v, 8);
+    v += __shfl_xor(v, 16);
+    v += __shfl_xor(v, 32);
+    return v;
+}
+
+// Layer 5: dW5[t][ci] = sum_p dy[p] a4[p + off_t][ci] = sum_q dy[q - off_t] a4[q][ci],
+// db5 = sum_p dy[p]; partial layout [t][ci] then db5.
 __global__ __launch_bounds__(256) void k_out_bwd_w(const float *__restrict__ dy,
                                                    const u16 *__restrict__ a, int H, int W, int R,
                                                    float *__restrict__ part)
@@ -730,39 +810,66 @@ __global__ __launch_bounds__(256) void k_out_bwd_w(const float *__restrict__ dy,
     __shared__ float red[4][9 * CH + 1];
     const int segs = W / GSEG, rb = H / R;
     const int seg = blockIdx.x % segs, r = (blockIdx.x / segs) % rb, n = blockIdx.x / (segs * rb);
-    const int ci = threadIdx.x & 63, jg = threadIdx.x >> 6;
-    const int xs0 = seg * GSEG + 16 * jg;
-    float s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, sb = 0.f;
-    for (int yy = r * R; yy < r * R + R; ++yy) {
-        const size_t rows[3] = {((size_t)n * H + wrap(yy - 1, H)) * W, ((size_t)n * H + yy) * W,
-                                ((size_t)n * H + wrap(yy + 1, H)) * W};
-        // window: v[dy][dx] = a[yy + dy - 1][xx + dx - 1][ci]
-        float v[3][3];
+    const int c8 = 8 * (threadIdx.x & 7), px = threadIdx.x >> 3, wv = threadIdx.x >> 6;
+    float s[9][8], sb = 0.f;
 #pragma unroll
-        for (int dy = 0; dy < 3; ++dy)
+    for (int t = 0; t < 9; ++t)
 #pragma unroll
-            for (int dx = 0; dx < 2; ++dx)
-                v[dy][dx + 1] = bf2f(a[(rows[dy] + wrap(xs0 + dx - 1, W)) * CH + ci]);
-        // (unrolled: the row's 48 + 16 loads in flight together instead of
-        // four per pixel in turn)
+        for (int k = 0; k < 8; ++k) s[t][k] = 0.f;
+    const int y0 = r * R;
+    for (int h = 0; h < 2; ++h) {
+        const int xx = seg * GSEG + 32 * h + px;
+        const int xs[3] = {wrap(xx - 1, W), xx, wrap(xx + 1, W)};
+        const float *dn = dy + (size_t)n * H * W;
+        const u16 *an = a + ((size_t)n * H * W + xx) * CH + c8;
+        // d[j][i]: dy at row y - 1 + j, column xx - 1 + i
+        float d[3][3];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int xx = xs0 + j;
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int dy = 0; dy < 3; ++dy) {
-                v[dy][0] = v[dy][1];
-                v[dy][1] = v[dy][2];
-                v[dy][2] = bf2f(a[(rows[dy] + wrap(xx + 1, W)) * CH + ci]);
+            for (int i = 0; i < 3; ++i) d[j + 1][i] = dn[(size_t)wrap(y0 - 1 + j, H) * W + xs[i]];
+        for (int yb = y0; yb < y0 + R; yb += GR) { // GR rows' loads in flight together
+            uint4 v[GR];
+            float e[GR][3];
+#pragma unroll
+            for (int k = 0; k < GR; ++k) {
+                v[k] = *reinterpret_cast<const uint4 *>(an + (size_t)(yb + k) * W * CH);
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    e[k][i] = dn[(size_t)wrap(yb + k + 1, H) * W + xs[i]];
             }
-            const float d = dy[(size_t)n * H * W + (size_t)yy * W + xx];
-            sb += d;
 #pragma unroll
-            for (int t = 0; t < 9; ++t) s[t] += d * v[t / 3][t % 3];
+            for (int k = 0; k < GR; ++k) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    d[0][i] = d[1][i];
+                    d[1][i] = d[2][i];
+                    d[2][i] = e[k][i];
+                }
+                sb += d[1][1];
+                float f[8];
+                unpack_bf16x8(v[k], f);
+#pragma unroll
+                for (int t = 0; t < 9; ++t) { // q - off_t: row y + 1 - t / 3, column x + 1 - t % 3
+                    const float g = d[2 - t / 3][2 - t % 3];
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) s[t][c] += g * f[c];
+                }
+            }
         }
     }
 #pragma unroll
-    for (int t = 0; t < 9; ++t) red[jg][t * CH + ci] = s[t];
-    if (ci == 0) red[jg][9 * CH] = sb;
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s[t][k] = add_columns(s[t][k]);
+    sb = add_columns(sb);
+    if ((threadIdx.x & 63) < 8) {
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) red[wv][t * CH + c8 + k] = s[t][k];
+        if (c8 == 0) red[wv][9 * CH] = sb;
+    }
     __syncthreads();
     float *pb = part + (size_t)blockIdx.x * (9 * CH + 1);
     for (int i = threadIdx.x; i < 9 * CH + 1; i += 256)
@@ -772,6 +879,7 @@ __global__ __launch_bounds__(256) void k_out_bwd_w(const float *__restrict__ dy,
 // Layer 0: dW0[t][ci][co] = sum_p xs_ci[p + off_t] dZ0[p][co] (xs the scaled,
 // BF16-rounded input), db0[co] = sum_p dZ0[p][co]; partial layout
 // [(t, ci)][co] then db0. The inputs go through LDS GR rows at a time.
+// (Four channels and 16 lanes a pixel: eight channels' 152 sums spill.)
 __global__ __launch_bounds__(256) void k_in_bwd_w(const float *__restrict__ x0,
                                                   const float *__restrict__ x1, long long sN,
                                                   int ld, float s0, float s1,
@@ -783,11 +891,15 @@ __global__ __launch_bounds__(256) void k_in_bwd_w(const float *__restrict__ x0,
     __shared__ float red[4][NO];
     const int segs = W / GSEG, rb = H / R;
     const int seg = blockIdx.x % segs, r = (blockIdx.x / segs) % rb, n = blockIdx.x / (segs * rb);
-    const int co = threadIdx.x & 63, jg = threadIdx.x >> 6;
+    const int c4 = 4 * (threadIdx.x & 15), px = threadIdx.x >> 4, wv = threadIdx.x >> 6;
     const int xb = seg * GSEG;
-    float s[9][2], sb = 0.f;
+    float s[18][4], sb[4];
 #pragma unroll
-    for (int t = 0; t < 9; ++t) s[t][0] = s[t][1] = 0.f;
+    for (int k = 0; k < 4; ++k) {
+        sb[k] = 0.f;
+#pragma unroll
+        for (int t = 0; t < 18; ++t) s[t][k] = 0.f;
+    }
     for (int y0 = r * R; y0 < r * R + R; y0 += GR) {
         __syncthreads(); // the previous rows' reads are done
         for (int q = threadIdx.x; q < (GR + 2) * (GSEG + 2); q += 256) {
@@ -797,28 +909,50 @@ __global__ __launch_bounds__(256) void k_in_bwd_w(const float *__restrict__ x0,
             xs[1][i][j] = bfr(s1 * x1[o]);
         }
         __syncthreads();
-        // (unrolled: the dZ loads of the GR rows in flight together instead
-        // of one per pixel in turn)
+#pragma unroll 1
+        for (int h = 0; h < 4; ++h) {
+            const int j = 16 * h + px;
+            const u16 *zn = dz + (((size_t)n * H + y0) * W + xb + j) * CH + c4;
+            uint2 v[GR]; // the GR rows' loads in flight together
 #pragma unroll
-        for (int i = 0; i < GR; ++i)
+            for (int i = 0; i < GR; ++i)
+                v[i] = *reinterpret_cast<const uint2 *>(zn + (size_t)i * W * CH);
 #pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-                const int j = 16 * jg + jj;
-                const float d = bf2f(dz[(((size_t)n * H + y0 + i) * W + xb + j) * CH + co]);
-                sb += d;
+            for (int i = 0; i < GR; ++i) {
+                const float f[4] = {bf2f((u16)(v[i].x & 0xffffu)), bf2f((u16)(v[i].x >> 16)),
+                                    bf2f((u16)(v[i].y & 0xffffu)), bf2f((u16)(v[i].y >> 16))};
+#pragma unroll
+                for (int k = 0; k < 4; ++k) sb[k] += f[k];
 #pragma unroll
                 for (int t = 0; t < 9; ++t) {
-                    s[t][0] += xs[0][i + t / 3][j + t % 3] * d;
-                    s[t][1] += xs[1][i + t / 3][j + t % 3] * d;
+                    const float g0 = xs[0][i + t / 3][j + t % 3], g1 = xs[1][i + t / 3][j + t % 3];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        s[2 * t][k] += g0 * f[k];
+                        s[2 * t + 1][k] += g1 * f[k];
+                    }
                 }
             }
+        }
     }
+    auto add = [](float v) { // over the wave's four pixel columns
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
 #pragma unroll
-    for (int t = 0; t < 9; ++t) {
-        red[jg][(2 * t + 0) * CH + co] = s[t][0];
-        red[jg][(2 * t + 1) * CH + co] = s[t][1];
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+        for (int t = 0; t < 18; ++t) s[t][k] = add(s[t][k]);
+        sb[k] = add(sb[k]);
     }
-    red[jg][9 * 2 * CH + co] = sb;
+    if ((threadIdx.x & 63) < 16) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+#pragma unroll
+            for (int t = 0; t < 18; ++t) red[wv][t * CH + c4 + k] = s[t][k];
+            red[wv][18 * CH + c4 + k] = sb[k];
+        }
+    }
     __syncthreads();
     float *pb = part + (size_t)blockIdx.x * NO;
     for (int i = threadIdx.x; i < NO; i += 256) pb[i] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
@@ -1021,7 +1155,7 @@ int forward(s2d_cnn *c, int B, const float *x0, const float *x1, long long sN, i
                (const u16 *)nullptr, keep_z ? c->z[l] : nullptr, c->a[l], 0);
         CNN_TRY(launched(c, "k_conv64"));
     }
-    hipLaunchKernelGGL(k_conv_out, dim3(W / 32, B * H), dim3(256), 0, c->stream, c->a[NMID],
+    hipLaunchKernelGGL(k_conv_out, dim3(W / 32, B * H / CO_ROWS), dim3(256), 0, c->stream, c->a[NMID],
                        c->P, c->y, B, H, W);
     return launched(c, "k_conv_out");
 }
@@ -1049,8 +1183,8 @@ int backward(s2d_cnn *c, int B, const float *x0, const float *x1, long long sN, 
                        rth, c->part);
     CNN_TRY(launched(c, "k_out_bwd_w"));
     CNN_TRY(reduce(nth, 9 * CH + 1, c->G + OFF_W5));
-    hipLaunchKernelGGL(k_out_bwd_data, dim3((unsigned)((npx + OB_PX - 1) / OB_PX)), dim3(256), 0,
-                       c->stream, c->dy, c->P, c->z[NMID], c->dz[0], B, H, W);
+    hipLaunchKernelGGL(k_out_bwd_data, dim3(W / 32, B * H / OB_ROWS), dim3(256), 0, c->stream,
+                       c->dy, c->P, c->z[NMID], c->dz[0], B, H, W);
     CNN_TRY(launched(c, "k_out_bwd_data"));
     int cur = 0;
     const int rdw = dw_rows(B, H, W, width_of(c, 512)), ndw = (int)dw_blocks(B, H, W, width_of(c, 512));
