@@ -280,13 +280,14 @@ int s2d_set_taylor_green(s2d_ctx *ctx);
  * per pass of the fused step, one of the kernel variants compiled for the
  * context's padded size (index 0 is the default; the single-run sizes
  * Np = 768, 1536, 3072 carry alternatives: the other twiddle batching, the
- * other pass B row pairing and, in FP32, 24 elements per lane for passes A
- * and C), and whether multi-step calls replay one captured step (hipGraph).
+ * other pass B row pairing and, in FP32, the other number of elements per
+ * lane for passes A and C), and whether calls of a few steps replay one
+ * captured step (hipGraph; longer ones launch ahead of the device).
  * Every variant computes the same mathematics; results differ at rounding
  * level only. */
 typedef struct s2d_schedule {
     int pass_a, pass_b, pass_c; /* variant index of each pass */
-    int step_graph;             /* 1: multi-step calls replay a captured step */
+    int step_graph;             /* 1: short calls replay a captured step */
     double step_us;             /* s2d_tune: measured microseconds per step */
     double default_us;          /* s2d_tune: the default schedule's, eager */
     int candidates, rejected;   /* s2d_tune: schedules timed / failing the check */

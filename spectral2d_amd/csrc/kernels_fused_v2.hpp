@@ -75,8 +75,11 @@ struct WaveCfg {
     static constexpr int THR3_A = sizeof(T) == 4 && TG > 12 ? 384 : 192;
     static constexpr int LPB_A = !P2 ? (TG >= 192 ? 2 : THR3_A / TG)
                                  : TG >= 256 ? (sizeof(T) == 4 ? 2 : 1) : THR_P2 / TG;
-    // pass B: two rows per lane group from Np = 1536 up (passB_pair)
-    static constexpr bool PAIR_B = (NP >= 1536) != ((V & VAR_PAIR) != 0);
+    // pass B: two rows per lane group from Np = 1536 up (passB_pair); one in
+    // FP64 at 3072, where 1536 groups fill the chip either way and the single
+    // row's fewer live registers win (step 747 -> 720 us; at 1536 163 -> 180)
+    static constexpr bool PAIR_B = (NP >= 1536 && !(sizeof(T) == 8 && NP >= 3072)) !=
+                                   ((V & VAR_PAIR) != 0);
     static constexpr int LPB_B = PAIR_B ? 2 : !P2 ? 192 / TG
                                  : TG >= 128 && sizeof(T) == 8 ? 1 : TG >= 256 ? 2 : THR_P2 / TG;
     static constexpr int THR_B = PAIR_B ? LPB_B * TG / 2 : LPB_B * TG; // lanes per block
@@ -114,7 +117,7 @@ struct WaveCfg {
     // less than loading the final ones too)
     static constexpr int TW_PRE_A0 =
         TAB ? TW_EARLY
-            : sizeof(T) == 8 ? (TW_EARLY | TW_FINAL_POW) : TG >= 128 ? TW_ALL : TW_FINAL_POW;
+            : sizeof(T) == 8 ? (TW_EARLY | TW_FINAL_POW) : NP >= 1536 ? TW_ALL : TW_FINAL_POW;
     static constexpr int TW_PRE_A = (V & VAR_TW_A) ? tw_flip(TW_PRE_A0) : TW_PRE_A0;
     // pass B: the lane's twiddles stay in registers for all of its row
     // transforms; FP64 has room next to the data (256 VGPRs) for the

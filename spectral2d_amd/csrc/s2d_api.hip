@@ -757,7 +757,8 @@ int launch2_passC(s2d_ctx *c, const cpx<T> *Wst, cpx<T> *Wout, const StageArgs &
 // twiddle mode for every pass, the other pass B row pairing, (FP32) 24
 // elements per lane for passes A and C, and pass A with the three fields of
 // a tile in one block. (24 per lane spills FP64 passes and every pass B.)
-// The ensemble's smaller sizes have the default only.
+// The ensemble's smaller sizes have the default only. Index 0 of pass A is
+// 24 per lane at FP32 Np = 3072 (e24_a), whose index 2 is then 12.
 template <typename T, int NP>
 constexpr bool tune_size()
 {
@@ -773,13 +774,26 @@ constexpr int n_variants()
     else return sizeof(T) == 4 ? 3 : 2;
 }
 
+// Pass A with 24 elements per lane by default: FP32 at Np = 1536 and 3072,
+// where a column then spans one and two waves instead of two and four (fewer
+// exchanges through LDS, fewer waves to wait for at each): the step takes 127
+// instead of 132 us and 352 instead of 364, at the same error against 64 bits
+// (1.12e-7 to 1.27e-7, to 1 % the same). At 768 its 384 columns are too few
+// waves.
+template <typename T, int NP>
+constexpr bool e24_a()
+{
+    return sizeof(T) == 4 && (NP == 1536 || NP == 3072);
+}
+
 template <typename T, int NP, int P, int I>
 constexpr int variant_bits()
 {
     static_assert(I < n_variants<T, NP, P>(), "no such variant");
-    if constexpr (I == 0) return 0;
-    else if constexpr (P == 0)
-        return I == 1 ? VAR_TW_A : (I == 2 && sizeof(T) == 4) ? VAR_E24 : VAR_FUSE_A;
+    if constexpr (P == 0 && sizeof(T) == 4 && (I == 0 || I == 2))
+        return (I == 2) != e24_a<T, NP>() ? VAR_E24 : 0;
+    else if constexpr (I == 0) return 0;
+    else if constexpr (P == 0) return I == 1 ? VAR_TW_A : VAR_FUSE_A;
     else if constexpr (P == 1) return I == 1 ? VAR_TW_B : VAR_PAIR;
     else return I == 1 ? VAR_TW_C : VAR_E24;
 }
@@ -898,7 +912,7 @@ int fused_vmax(s2d_ctx *c, double *vmax)
     int r = S2D_ERR_UNSUPPORTED;
     const cpx<T> *Wn = (const cpx<T> *)c->Wn;
     if (const int np = wave_np<T>(c)) {
-        S2D_WAVE_SWITCH(T, np, r = (launch2_passA<T, NP>(c, Wn, 1));
+        S2D_WAVE_SWITCH(T, np, r = (launch2_passA<T, NP, variant_bits<T, NP, 0, 0>()>(c, Wn, 1));
                         if (!r) r = (launch2_passB<T, NP>(c, 0, 1)))
     } else switch (EC) {
     case 12: r = launch_passA<T, 12>(c, Wn, 1); if (!r) r = launch_passB<T, 12>(c, 0, 1); break;
@@ -1182,9 +1196,8 @@ void drop_step_graph(s2d_ctx *c)
     c->step_graph = nullptr;
 }
 
-// Multi-step calls of a single run with the compiled wave kernels replay
-// one captured step (hipGraph): the step's 9 launches then go out without
-// host round trips between them. The graph is re-captured when an argument
+// One captured step (hipGraph), replayed: its 9 launches go out in one host
+// call. The graph is re-captured when an argument
 // baked into it changes (nu, dt, cfl, the forcing buffer, the schedule).
 // Inside a timing session the sampled steps run eagerly with their events.
 template <typename T>
@@ -1776,7 +1789,17 @@ int s2d_rk3_steps(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
     }
     S2D_TRY(ensure_compact(c));
     if (nsteps == 0) return sync(c);
+    // Short calls of a single run with the compiled wave kernels replay one
+    // captured step. A replay starts about 10 us sooner than nine launches
+    // do, but leaves about 4.5 us of gap before the next replay (launches that
+    // run ahead of the device leave none), so calls of 4 steps and more launch
+    // them one by one: us per call of 1 / 2 / 8 steps, replayed / launched,
+    // FP64: N = 96 79 / 90, 136 / 144, 474 / 461; N = 512 121 / 129,
+    // 218 / 223, 803 / 785; N = 1024 (10 steps) 1672 / 1627. A step at N = 64
+    // (44 us) is as short as its nine launches take on a slow host (8 steps
+    // 398 / 418, on a fast one 400 / 386) and is always replayed.
     const bool graphed = c->step_graph_on && c->nruns == 1 &&
+                         (nsteps < 4 || c->g.nxG < 144) &&
                          (c->precision == S2D_FP64 ? wave_np<double>(c) : wave_np<float>(c)) != 0;
     if (graphed)
         S2D_TRY(S2D_DISPATCH_T(c, fused_steps_graphed, nsteps, nu, dt, cfl));
