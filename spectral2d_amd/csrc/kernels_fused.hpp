@@ -410,10 +410,12 @@ __device__ __forceinline__ void diag_mode(cpx<T> w, int kx, int ky, int kxMG, do
 __device__ __forceinline__ void diag_block(const double (&a)[5], double *__restrict__ part)
 {
     __shared__ double sh[5][256];
+#pragma unroll
     for (int q = 0; q < 5; ++q) sh[q][threadIdx.x] = a[q];
     __syncthreads();
     for (int o = blockDim.x / 2; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) {
+#pragma unroll
             for (int q = 0; q < 5; ++q) {
                 if (q == 3)
                     sh[q][threadIdx.x] = fmax(sh[q][threadIdx.x], sh[q][threadIdx.x + o]);
@@ -465,27 +467,20 @@ __global__ void k_diag_runs(const cpx<T> *__restrict__ Wc, long long sW, FusedDi
     diag_block(a, part + ((size_t)blockIdx.y * gridDim.x + blockIdx.x) * 5);
 }
 
-// Run blockIdx.x's five values from its nb blocks' partials, in block order.
+// Run blockIdx.x's five values from its nb blocks' partials: the threads' strided
+// sums in the blocks' fixed tree. Bound by latency (512 blocks: 4 us; one
+// chain of additions in block order took 16).
 static __global__ __launch_bounds__(256) void k_diag_sum(const double *__restrict__ part, int nb,
                                                   double *__restrict__ out)
 {
-    __shared__ double sh[256 * 5];
     part += (size_t)blockIdx.x * nb * 5;
-    const int q = threadIdx.x;
-    double s = 0.0;
-    for (int b0 = 0; b0 < nb; b0 += 256) {
-        const int m = nb - b0 < 256 ? nb - b0 : 256;
-        __syncthreads();
-        for (int k = threadIdx.x; k < 5 * m; k += 256) sh[k] = part[(size_t)b0 * 5 + k];
-        __syncthreads();
-        if (q < 5)
-            for (int b = 0; b < m; ++b) {
-                const double x = sh[b * 5 + q];
-                if (q == 3) s = x > s ? x : s;
-                else s += x;
-            }
-    }
-    if (q < 5) out[(size_t)blockIdx.x * 5 + q] = s;
+    double a[5] = {0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nb; b += 256)
+        for (int q = 0; q < 5; ++q) {
+            const double x = part[(size_t)b * 5 + q];
+            a[q] = q == 3 ? fmax(a[q], x) : a[q] + x;
+        }
+    diag_block(a, out + (size_t)blockIdx.x * 5);
 }
 
 } // namespace s2d

@@ -1051,16 +1051,19 @@ int spectrum_of(s2d_ctx *c, double nu, double *ek, int *cnt, double *tke, double
     const int nb = s2d_spectrum_bins(&g);
     double *d_ek = c->d_red; // nb sums, then nb counts
     int *d_cnt = reinterpret_cast<int *>(d_ek + nb);
-    auto shells = [&](auto uv, auto zero) {
+    auto shells = [&](auto uv, auto zero, auto idx) {
         using T = decltype(zero);
-        hipLaunchKernelGGL((k_spectrum<T, decltype(uv)::value>), dim3(nb), dim3(256), 0, c->stream,
-                           F<T>(c, fa), F<T>(c, fb < 0 ? fa : fb), g.cISize, g.nyG, g.kxMG,
-                           g.kyMG, c->xMaskBool, c->yMaskBool, d_ek, d_cnt);
+        hipLaunchKernelGGL((k_spectrum<T, decltype(uv)::value, decltype(idx)>),
+                           dim3((nb + 63) / 64 * 64), dim3(256), 0, c->stream, F<T>(c, fa),
+                           F<T>(c, fb < 0 ? fa : fb), g.cISize, g.nyG, g.kxMG, g.kyMG,
+                           c->xMaskBool, c->yMaskBool, nb, d_ek, d_cnt);
     };
-    if (c->precision == S2D_FP64)
-        fb < 0 ? shells(std::false_type{}, 0.0) : shells(std::true_type{}, 0.0);
-    else
-        fb < 0 ? shells(std::false_type{}, 0.0f) : shells(std::true_type{}, 0.0f);
+    auto spectra = [&](auto zero, auto idx) {
+        fb < 0 ? shells(std::false_type{}, zero, idx) : shells(std::true_type{}, zero, idx);
+    };
+    const bool small = nb < 65535;
+    if (c->precision == S2D_FP64) small ? spectra(0.0, 0u) : spectra(0.0, 0ull);
+    else small ? spectra(0.0f, 0u) : spectra(0.0f, 0ull);
     S2D_LAUNCHED(c, "k_spectrum");
     std::vector<double> h((size_t)nb + (nb + 1) / 2);
     S2D_HIP(c, hipMemcpyAsync(h.data(), d_ek, (sizeof(double) + sizeof(int)) * nb,
