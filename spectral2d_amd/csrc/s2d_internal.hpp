@@ -87,6 +87,9 @@ struct s2d_ctx {
     // index of passes A, B, C among those compiled for the padded size, and
     // whether multi-step calls replay a captured step (hipGraph)
     int var[3] = {0, 0, 0};
+    // page-locked staging of small transfers (stage_bytes), each used up
+    // before its call returns; null where it could not be had
+    char *stage = nullptr;
     bool step_graph_on = true;
     hipGraphExec_t step_graph = nullptr;
     double sg_nu = 0.0, sg_dt = 0.0, sg_cfl = 0.0; // the captured step's arguments
