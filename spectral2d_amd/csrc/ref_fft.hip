@@ -520,6 +520,68 @@ k_rhs_rows(cpx<T> *u, cpx<T> *v, cpx<T> *w, int cI, int nin, int nout, int ny,
     row_r2c<T, H>(ww, w + at, t, no, w0, slice, gt);
 }
 
+// The same rows with a lane group to a field: u w, v w and w's round trip run
+// beside each other, each group transforming w itself, so that a row's chain
+// is three transforms instead of six for half as much work again. For grids
+// whose k_rhs_rows blocks leave CUs idle, where that chain is the time
+// (rhs_rows_split; the same arithmetic, to the bit).
+template <typename T, int H>
+struct RowSplitCfg {
+    using C = RowCfg<T, H>;
+    static constexpr int RB = C::P2 ? (C::TG >= 64 ? 1 : 64 / C::TG) : C::TG >= 96 ? 1 : 96 / C::TG;
+    static constexpr int THR = 3 * RB * C::TG;
+};
+
+template <typename T, int H>
+__global__ __launch_bounds__((RowSplitCfg<T, H>::THR)) void
+k_rhs_rows_split(cpx<T> *u, cpx<T> *v, cpx<T> *w, int cI, int nin, int nout, int ny,
+                 const cpx<T> *__restrict__ tw, const cpx<T> *__restrict__ twx)
+{
+#pragma clang fp contract(off)
+    using C = RowCfg<T, H>;
+    constexpr int RB = RowSplitCfg<T, H>::RB;
+    __shared__ cpx<T> lds[3 * RB * C::SL];
+    const int gr = (int)threadIdx.x / C::TG, t = threadIdx.x % C::TG;
+    const int j0 = blockIdx.x * RB + gr % RB, field = gr / RB;
+    const int j = j0 < ny ? j0 : ny - 1; // (rows past the end repeat the last one, unstored)
+    const size_t at = (size_t)j * cI;
+    cpx<T> *slice = lds + gr * C::SL;
+    auto last = [&](const cpx<T> *f) { return nin > H ? f[H] : mk<T>((T)0, (T)0); };
+    cpx<T> *f = (field == 0 ? u : field == 1 ? v : w) + at;
+    cpx<T> ww[C::E], x[C::E];
+    row_load<T, H>(ww, w + at, t, nin);
+    row_load<T, H>(x, f, t, nin);
+    const cpx<T> lw = last(w + at), lf = last(f), w0 = twx[t];
+    RowTw<T, H> gt;
+    gt.load(tw, t);
+    row_c2r<T, H>(ww, lw, t, w0, slice, gt);
+    row_c2r<T, H>(x, lf, t, w0, slice, gt);
+#pragma unroll
+    for (int s = 0; s < C::E; ++s)
+        x[s] = field == 2 ? ww[s] : mk<T>(x[s].re * ww[s].re, x[s].im * ww[s].im);
+    __syncthreads(); // (every group has its w: the third may write it)
+    row_r2c<T, H>(x, f, t, j0 < ny ? nout : 0, w0, slice, gt);
+}
+
+// Rows by k_rhs_rows_split: while k_rhs_rows has no more than 128 blocks in FP64
+// and 384 in FP32. Past that the chip is full and the work added
+// costs more than the shorter chain gives. ComputeRHS, us, one group to a row /
+// one to a field, FP64: 64^2 35.3 / 32.6, 256^2 51.1 / 45.9, 384^2 (72 blocks)
+// 58.3 / 55.3, 512 x 256 (96) 57.3 / 51.6, 512^2 (192) 67.7 / 69.9, 256 x 1024
+// (192) 72.0 / 74.5; FP32: 64^2 31.8 / 27.9, 512^2 57.4 / 54.8, 512 x 1024 (384)
+// 74.2 / 72.2.
+template <typename T, int H>
+constexpr bool row_split_len()
+{
+    return H <= 384;
+}
+template <typename T, int H>
+bool rhs_rows_split(int ny)
+{
+    constexpr int RB = RowCfg<T, H>::RB;
+    return row_split_len<T, H>() && (ny + RB - 1) / RB <= (sizeof(T) == 8 ? 128 : 384);
+}
+
 // f(std::integral_constant<int, n>) for a compiled length.
 template <typename F>
 bool with_length(int n, F &&f)
@@ -598,11 +660,21 @@ void ref_rhs(hipStream_t st, const RefGrid &g, const cpx<T> *psi_in, cpx<T> *u, 
     with_length(g.h, [&](auto n) {
         constexpr int H = decltype(n)::value;
         if constexpr (H <= 1536) {
+            const cpx<T> *th = static_cast<const cpx<T> *>(g.tw_h);
+            const cpx<T> *tx = static_cast<const cpx<T> *>(g.tw_x);
+            if constexpr (row_split_len<T, H>()) {
+                if (rhs_rows_split<T, H>(g.ny)) {
+                    constexpr int RS = RowSplitCfg<T, H>::RB;
+                    hipLaunchKernelGGL((k_rhs_rows_split<T, H>), dim3((g.ny + RS - 1) / RS),
+                                       dim3(RowSplitCfg<T, H>::THR), 0, st, u, v, w, g.cI, nin,
+                                       nout, g.ny, th, tx);
+                    return;
+                }
+            }
             constexpr int RB = RowCfg<T, H>::RB;
             hipLaunchKernelGGL((k_rhs_rows<T, H>), dim3((g.ny + RB - 1) / RB),
-                               dim3(RowCfg<T, H>::THR), 0, st, u, v, w, g.cI, nin, nout, g.ny,
-                               static_cast<const cpx<T> *>(g.tw_h),
-                               static_cast<const cpx<T> *>(g.tw_x));
+                               dim3(RowCfg<T, H>::THR), 0, st, u, v, w, g.cI, nin, nout, g.ny, th,
+                               tx);
         }
     });
     const RhsArgs<T> a = {u,    v,    w,        dW,       w0,    out,    psi, g.cI,
