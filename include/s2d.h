@@ -280,8 +280,8 @@ int s2d_set_taylor_green(s2d_ctx *ctx);
  * per pass of the fused step, one of the kernel variants compiled for the
  * context's padded size (index 0 is the default; the single-run sizes
  * Np = 768, 1536, 3072 carry alternatives: the other twiddle batching, the
- * other pass B row pairing and, in FP32, the other number of elements per
- * lane for passes A and C), and whether calls of a few steps replay one
+ * other pass B row pairing and, in FP32, other elements per lane or
+ * twiddles for passes A and C), and whether calls of a few steps replay one
  * captured step (hipGraph; longer ones launch ahead of the device).
  * Every variant computes the same mathematics; results differ at rounding
  * level only. */

@@ -804,7 +804,9 @@ int launch2_passC(s2d_ctx *c, const cpx<T> *Wst, cpx<T> *Wout, const StageArgs &
 // elements per lane for passes A and C, and pass A with the three fields of
 // a tile in one block. (24 per lane spills FP64 passes and every pass B.)
 // The ensemble's smaller sizes have the default only. Index 0 of pass A is
-// 24 per lane at FP32 Np = 3072 (e24_a), whose index 2 is then 12.
+// 24 per lane in FP32 from Np = 1536 (e24_a); index 2 is 24 there too, with
+// the other twiddle mode (at 1536, with B and C flipped, 120 us a step
+// instead of 126, at twice the error: for the tuner to take).
 template <typename T, int NP>
 constexpr bool tune_size()
 {
@@ -836,10 +838,11 @@ template <typename T, int NP, int P, int I>
 constexpr int variant_bits()
 {
     static_assert(I < n_variants<T, NP, P>(), "no such variant");
-    if constexpr (P == 0 && sizeof(T) == 4 && (I == 0 || I == 2))
-        return (I == 2) != e24_a<T, NP>() ? VAR_E24 : 0;
+    if constexpr (P == 0 && e24_a<T, NP>() && (I == 0 || I == 2))
+        return I == 0 ? VAR_E24 : VAR_E24 | VAR_TW_A;
     else if constexpr (I == 0) return 0;
-    else if constexpr (P == 0) return I == 1 ? VAR_TW_A : VAR_FUSE_A;
+    else if constexpr (P == 0)
+        return I == 1 ? VAR_TW_A : (I == 2 && sizeof(T) == 4) ? VAR_E24 : VAR_FUSE_A;
     else if constexpr (P == 1) return I == 1 ? VAR_TW_B : VAR_PAIR;
     else return I == 1 ? VAR_TW_C : VAR_E24;
 }

@@ -1,6 +1,6 @@
 """The default schedule's choices on the GPU: calls that replay a captured
 step and calls that launch theirs one by one give the same bits, and the
-default kernels of the largest sizes agree with the variants they stand for."""
+default kernels of the largest sizes agree with their alternatives."""
 import numpy as np
 import pytest
 
@@ -31,7 +31,7 @@ def test_short_and_long_calls_equal_eager(N, prec):
 
 @pytest.mark.parametrize("N,prec,sched", [(1024, FP32, (2, 0, 0)), (2048, FP32, (2, 0, 0)),
                                           (2048, FP64, (0, 2, 0))])
-def test_default_agrees_with_the_kernel_it_replaced(N, prec, sched):
+def test_default_agrees_with_its_alternative(N, prec, sched):
     """Same mathematics, other order of rounding: the variants' tolerances
     (1e-12, 1e-5), and not the same kernel (the bits differ)."""
     print(f"[schedule] N={N} precision={prec} default vs {sched}", flush=True)
