@@ -7,13 +7,15 @@
 // Elements per lane: 12 in both precisions (a 1536-point transform spans
 // two waves with four LDS exchanges; 24 per lane would fit it in one wave
 // with two exchanges, but at about twice the registers per wave, which
-// spills pass B and halves the waves in flight).
+// spills pass B and halves the waves in flight; FP32 pass A, whose tiles are
+// the smallest, gains by it at Np = 1536 and 3072).
 //
 //  A  one lane group per (field, kx): u_hat, v_hat or w_hat of a column,
 //     inverse transform along y. A block holds LPB adjacent columns of one
 //     field; it stages them in LDS and stores the G rows (G[y*KG + kx]) as
 //     LPB-element contiguous segments.
-//  B  one lane group per row y, or per two rows from Np = 1536 up
+//  B  one lane group per row y, or per two rows from Np = 1536 up (FP64 at
+//     3072: one)
 //     (contiguous loads of the G rows): w from its Hermitian spectrum (two
 //     rows' w from one transform of w_a + i w_b), u + i v (two-for-one), the
 //     products (u w + i v w) in registers, one forward transform, the uw /
@@ -110,8 +112,9 @@ struct WaveCfg {
     // pass A: FP64 loads its early-pass twiddles in one batch (1.3 % less
     // time at Np = 1536 than all in one batch at two waves) and forms the
     // final pass's as powers of W^t (6 % less time than loading them per
-    // use); FP32 loads all in one batch for the two-wave groups
-    // (Np >= 1536: 5 % less time), and for the ensemble's sizes loads the
+    // use); FP32 loads all in one batch from Np = 1536
+    // up (5 % less time with 12 elements per lane; with 24, powers are 3 %
+    // faster still and double the error), and for the ensemble's sizes loads the
     // early-pass ones per pass and forms the final pass's as powers (4 %
     // less time for the mixed ensemble than all in one batch, then 2.6 %
     // less than loading the final ones too)
