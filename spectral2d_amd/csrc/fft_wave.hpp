@@ -159,10 +159,26 @@ constexpr double cos15(int a)
 }
 constexpr double sin15(int a) { return cos15(a - 6); }
 
+// What cos(15 a degrees) has beyond its FP64 value where that is +-sqrt(3)/2,
+// else 0: the one constant of radix 12 that is not exact, and FP64 rounds it
+// by 0.45 of its last place.
+constexpr double cos15_low(int a)
+{
+    constexpr double low = 5.01754211090345140e-17; // (long double is double on the device)
+    const double c = cos15(a);
+    return c == kCos15[2] ? low : c == -kCos15[2] ? -low : 0.0;
+}
+
 // x * exp(D i 2 pi e / N) for compile-time e and N | 24 (D = -1 forward,
 // +1 inverse): multiples of a quarter turn are exact swaps and negations,
 // the rest one complex product with constants.
-template <typename T, int D, int N, int e>
+// ACC (FP64): sqrt(3)/2 in two terms, one FMA more. As a single constant in
+// every pass its rounding adds up: error of a transform of length 144 / 1152
+// and back 2.83e-16 / 3.07e-16, in two terms here and in radix 3 2.36e-16 /
+// 2.70e-16 (the runtime plans, whose table twiddles all round differently,
+// 2.57e-16 / 2.86e-16); IntegrateOneStep at 96 / 768 / 1024 97 -> 101, 238 ->
+// 242 and 334 -> 336 us.
+template <typename T, int D, int N, int e, bool ACC = false>
 __device__ __forceinline__ cpx<T> twiddle_const(cpx<T> x)
 {
     static_assert(24 % N == 0, "constant twiddles cover sizes dividing 24");
@@ -176,17 +192,42 @@ __device__ __forceinline__ cpx<T> twiddle_const(cpx<T> x)
         return sg > 0 ? mk<T>(-x.im, x.re) : mk<T>(x.im, -x.re);
     } else {
         constexpr T c = (T)cos15(a), sn = (T)(D * sin15(a));
-        return mul(x, mk<T>(c, sn));
+        if constexpr (ACC && sizeof(T) == 8 && cos15_low(a) != 0.0) {
+            constexpr T cl = (T)cos15_low(a);
+            return mk<T>(fma(x.re, c, fma(x.re, cl, -(x.im * sn))),
+                         fma(x.im, c, fma(x.im, cl, x.re * sn)));
+        } else if constexpr (ACC && sizeof(T) == 8 && cos15_low(a - 6) != 0.0) {
+            constexpr T sl = (T)(D * cos15_low(a - 6));
+            return mk<T>(fma(-x.im, sn, fma(-x.im, sl, x.re * c)),
+                         fma(x.re, sn, fma(x.re, sl, x.im * c)));
+        } else {
+            return mul(x, mk<T>(c, sn));
+        }
     }
+}
+
+// Radix 3 with sqrt(3)/2 in two terms (see twiddle_const).
+template <int D>
+__device__ __forceinline__ void dft3_acc(cpx<double> *a)
+{
+    constexpr double h = D < 0 ? cos15(2) : -cos15(2), l = D < 0 ? cos15_low(2) : -cos15_low(2);
+    const cpx<double> t1 = add(a[1], a[2]), q = sub(a[1], a[2]);
+    const cpx<double> t2 = mk(a[0].re - 0.5 * t1.re, a[0].im - 0.5 * t1.im);
+    const cpx<double> t3 = mk(fma(q.re, h, q.re * l), fma(q.im, h, q.im * l));
+    a[0] = add(a[0], t1);
+    a[1] = mk(t2.re + t3.im, t2.im - t3.re);
+    a[2] = mk(t2.re - t3.im, t2.im + t3.re);
 }
 
 // In-register DFT of compile-time size N on a[0..N-1] (natural order in and
 // out). Base radices 2, 3, 4, 8; composite N = N1*N2 by Cooley-Tukey with
 // N1 the largest base radix dividing N, and compile-time twiddles.
-template <typename T, int N, int D>
+template <typename T, int N, int D, bool ACC = false>
 __device__ __forceinline__ void dft_ct(cpx<T> *a)
 {
-    if constexpr (N == 2 || N == 3 || N == 4 || N == 8) {
+    if constexpr (ACC && sizeof(T) == 8 && N == 3) {
+        dft3_acc<D>(a);
+    } else if constexpr (N == 2 || N == 3 || N == 4 || N == 8) {
         dft<T, N, D>(a);
     } else {
         constexpr int N1 = (N % 8 == 0) ? 8 : (N % 4 == 0) ? 4 : (N % 3 == 0) ? 3 : 2;
@@ -200,7 +241,7 @@ __device__ __forceinline__ void dft_ct(cpx<T> *a)
             dft<T, N1, D>(b);
             static_for<0, N1>([&](auto k1I) {
                 constexpr int k1 = decltype(k1I)::value;
-                y[n2 * N1 + k1] = twiddle_const<T, D, N, n2 * k1>(b[k1]);
+                y[n2 * N1 + k1] = twiddle_const<T, D, N, n2 * k1, ACC>(b[k1]);
             });
         });
 #pragma unroll
@@ -208,7 +249,7 @@ __device__ __forceinline__ void dft_ct(cpx<T> *a)
             cpx<T> c[N2];
 #pragma unroll
             for (int n2 = 0; n2 < N2; ++n2) c[n2] = y[n2 * N1 + k1];
-            dft_ct<T, N2, D>(c);
+            dft_ct<T, N2, D, ACC>(c);
 #pragma unroll
             for (int k2 = 0; k2 < N2; ++k2) a[k1 + N1 * k2] = c[k2];
         }
@@ -237,6 +278,9 @@ constexpr int early_tw_offset()
 // loads wait once per pass; batched ones hold registers for the whole
 // transform.
 constexpr int TW_EARLY = 1, TW_FINAL = 2, TW_ALL = 3, TW_FINAL_POW = 4;
+// bit 3: the constant twiddles inside the butterflies to more than FP64
+// (twiddle_const's ACC)
+constexpr int TW_ACC = 8;
 
 template <typename T, int E, int TG, int PRE = TW_ALL>
 struct GroupTw {
@@ -247,6 +291,7 @@ struct GroupTw {
     // multiplication each instead of a load (at most about E ulps apart
     // from the table's values)
     static constexpr bool PP = (PRE & TW_FINAL_POW) != 0;
+    static constexpr bool ACC = (PRE & TW_ACC) != 0;
     cpx<T> e[PE && NE > 0 ? NE : 1];
     cpx<T> f[PF ? E : 1];
     cpx<T> w1; // W^t (PP)
@@ -322,7 +367,7 @@ __device__ __forceinline__ void group_pass(cpx<T> (&v)[E], cpx<T> *lds, int t, c
 #pragma unroll
             for (int m = 1; m < R; ++m) a[m] = mul(a[m], dir<T, D>(g.template early<Ls, R>(m)));
         }
-        dft_ct<T, R, D>(a);
+        dft_ct<T, R, D, G::ACC>(a);
 #pragma unroll
         for (int m = 0; m < R; ++m) lds[LdsMap<TG>::idx_sum(ib, TG * q * R + m * Ls)] = a[m];
     }
@@ -362,7 +407,7 @@ __device__ __forceinline__ void final_pass(cpx<T> (&v)[E], const G &g)
 #pragma unroll
         for (int m = 1; m < E; ++m) v[m] = mul(v[m], dir<T, D>(g.final(m)));
     }
-    dft_ct<T, E, D>(v);
+    dft_ct<T, E, D, G::ACC>(v);
 }
 
 // Full transform of the group: on entry v[s] = x[t + TG*s], on exit
