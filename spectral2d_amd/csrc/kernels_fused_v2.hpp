@@ -32,6 +32,7 @@
 
 #include <type_traits>
 
+#include "exact_div.hpp"
 #include "fft_wave.hpp"
 #include "kernels_fused.hpp"
 
@@ -183,17 +184,6 @@ __device__ __forceinline__ double recip(double x)
     double r = __builtin_amdgcn_rcp(x);
     r = __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
     return __builtin_fma(r, __builtin_fma(-x, r, 1.0), r);
-}
-
-// x / 3, correctly rounded, without a division: q = RN(x * RN(1/3)) is
-// within one ulp of x/3, the remainder x - 3q is exact under FMA, and one
-// correction q + r * RN(1/3) rounds to RN(x/3) (Markstein's theorem).
-template <typename T>
-__device__ __forceinline__ T div3(T x)
-{
-    constexpr T y = (T)(1.0L / 3.0L);
-    const T q = x * y;
-    return fma(fma((T)-3, q, x), y, q);
 }
 
 // Where the padded index k = t + TG*S (0 <= t < TG) of a length-NP

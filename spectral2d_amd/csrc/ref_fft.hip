@@ -71,18 +71,6 @@ struct ColCfg {
     static constexpr int WPE = sizeof(T) == 8 ? (THR > 384 ? 2 : 3) : 4; // waves per SIMD
 };
 
-// x / d correctly rounded, with r = 1 / d rounded: q = x r is within one ulp,
-// its remainder is exact under FMA, and one correction rounds to x / d
-// (Markstein), at a quarter of the division's instructions. Values whose
-// remainder would underflow, and infinities, take the division (*odd).
-__device__ __forceinline__ double div_by(double x, double d, double r, bool *odd)
-{
-    const double q = x * r;
-    const double a = __builtin_fabs(x);
-    *odd |= !(a < 1.0e300) || (a < 1.0e-280 && a > 0.0);
-    return __builtin_fma(__builtin_fma(-d, q, x), r, q);
-}
-
 // v / norm of TransformR2C (src/Spectral.F90:761-762); FP32: div_real's
 // product with 1 / norm.
 template <typename T, int E>
@@ -230,14 +218,6 @@ struct RhsArgs {
     double norm, nu, dt;
     const cpx<T> *tw;
 };
-
-// x / 3 as div3, infinities kept.
-template <typename T>
-__device__ __forceinline__ T div3_any(T x)
-{
-    const T r = div3(x);
-    return x - x == (T)0 ? r : x;
-}
 
 // The forward column transforms of u w, v w and w, then per mode
 // TransformR2C's division, Truncate, DuDx / DuDy and dW = -u - v - nu k^2 w
