@@ -97,18 +97,25 @@ struct WaveCfg {
     // twice the data: two waves)
     static constexpr int WPE_A = (V & VAR_FUSE_A) ? (sizeof(T) == 8 ? 2 : 3)
                                  : E == 24 ? 2 : sizeof(T) == 8 ? 3 : 4;
-    static constexpr int WPE_C = E == 24 ? 2 : sizeof(T) == 8 ? 2 : TG <= 64 ? 5 : 4;
+    static constexpr int WPE_C = E == 24 ? 2 : sizeof(T) == 8 ? 2 : P2 && TG <= 64 ? 5 : 4;
     // pass C: the compact-state operands loaded ahead of the transform, and
     // the twiddles in one batch; FP64 and the ensemble's FP32 sizes form the
     // final pass's as powers of W^t (FP64: 168 VGPRs, three waves per SIMD,
     // 7 % less time at Np = 1536; FP32 Np <= 768: five waves, 7 % less
     // time for the mixed ensemble)
-    // (FP64 3*2^k: all from the table, as accurate as the runtime plans' to
-    // 20 %; powers took 4 % off these passes and added to the error)
-    static constexpr bool TAB = !P2 && sizeof(T) == 8;
+    // 3*2^k lanes: every pass takes its twiddles from the table, FP64 the
+    // constants of radix 12 in two terms (TW_ACC), pass A psi and pass C the
+    // normalisation as quotients and the last stage as a sum of thirds, so
+    // that the step is as accurate as on the runtime plans these kernels
+    // replaced. Four steps, error of w against 64 bits, plans / powers,
+    // reciprocals and a single third / so: FP64 N = 768 4.08e-16 / 4.74e-16 /
+    // 4.06e-16, FP32 N = 192 1.20e-7 / 1.90e-7 / 1.17e-7; a step of FP64 N = 96
+    // and 768 takes 164 and 408, 58 and 145, 61 and 160 us.
+    static constexpr bool TAB = !P2;
+    static constexpr int ACC = TAB && sizeof(T) == 8 ? TW_ACC : 0;
     static constexpr int TW_PRE_C0 =
         !TAB && (sizeof(T) == 8 || TG <= 64) ? (TW_EARLY | TW_FINAL_POW) : TW_ALL;
-    static constexpr int TW_PRE_C = (V & VAR_TW_C) ? tw_flip(TW_PRE_C0) : TW_PRE_C0;
+    static constexpr int TW_PRE_C = ((V & VAR_TW_C) ? tw_flip(TW_PRE_C0) : TW_PRE_C0) | ACC;
     static constexpr bool OPS_EARLY_C = true;
     // pass A: FP64 loads its early-pass twiddles in one batch (1.3 % less
     // time at Np = 1536 than all in one batch at two waves) and forms the
@@ -118,27 +125,27 @@ struct WaveCfg {
     // faster still and double the error), and for the ensemble's sizes loads the
     // early-pass ones per pass and forms the final pass's as powers (4 %
     // less time for the mixed ensemble than all in one batch, then 2.6 %
-    // less than loading the final ones too)
+    // less than loading the final ones too). 3*2^k lanes: FP64 and FP32 at
+    // Np = 2304 the early ones in a batch (2304 FP32: step 251 -> 241 us
+    // against all of them), else all
     static constexpr int TW_PRE_A0 =
-        TAB ? TW_EARLY
+        TAB ? (sizeof(T) == 8 || TG >= 192 ? TW_EARLY : TW_ALL)
             : sizeof(T) == 8 ? (TW_EARLY | TW_FINAL_POW) : NP >= 1536 ? TW_ALL : TW_FINAL_POW;
-    static constexpr int TW_PRE_A = (V & VAR_TW_A) ? tw_flip(TW_PRE_A0) : TW_PRE_A0;
+    static constexpr int TW_PRE_A = ((V & VAR_TW_A) ? tw_flip(TW_PRE_A0) : TW_PRE_A0) | ACC;
     // pass B: the lane's twiddles stay in registers for all of its row
     // transforms; FP64 has room next to the data (256 VGPRs) for the
     // early-pass ones only (measured: 9 % less time at Np = 1536 than
     // loading every twiddle per pass), and forms the final pass's as powers
     // of W^t (5 % less time than loading them)
-    static constexpr int TW_PRE_B0 = sizeof(T) == 4 ? TW_ALL : (TW_EARLY | TW_FINAL_POW);
-    static constexpr int TW_PRE_B = (V & VAR_TW_B) ? tw_flip(TW_PRE_B0) : TW_PRE_B0;
-    // (one row per lane group: every twiddle in one batch by default)
-    // (FP64 Np = 1152: powers, which fit three waves per SIMD, so that its
-    // 576 blocks run in one round: 22.9 -> 20.5 us)
-    static constexpr bool B3 = sizeof(T) == 8 && TG == 96;
-    static constexpr int TW_PRE_B10 = B3 ? (TW_EARLY | TW_FINAL_POW) : TW_ALL;
-    static constexpr int TW_PRE_B1 = (V & VAR_TW_B) ? tw_flip(TW_PRE_B10) : TW_PRE_B10;
+    static constexpr int TW_PRE_B0 = sizeof(T) == 4 || TAB ? TW_ALL : (TW_EARLY | TW_FINAL_POW);
+    static constexpr int TW_PRE_B = ((V & VAR_TW_B) ? tw_flip(TW_PRE_B0) : TW_PRE_B0) | ACC;
+    // (one row per lane group: every twiddle in one batch; FP64 Np = 1152 step
+    // 160 us, 168 with the early ones only in three waves per SIMD; Np = 2304,
+    // row pairs: 403, 418 with the early ones only)
+    static constexpr int TW_PRE_B1 = ((V & VAR_TW_B) ? tw_flip(TW_ALL) : TW_ALL) | ACC;
     // pass B holds w and u + i v; a multi-wave group needs more registers
     static constexpr int WPE_B =
-        B3 || (!P2 && sizeof(T) == 4 && !PAIR_B) ? 3
+        (!P2 && sizeof(T) == 4 && !PAIR_B) ? 3
         : (sizeof(T) == 8 || TG > 64 || E == 24) ? 2 : 3;
     static_assert(E * TG == NP && TG >= 2 && TG <= 256 &&
                       (P2 || (E == 12 && TG % 3 == 0 && ((TG / 3) & (TG / 3 - 1)) == 0)),
@@ -313,6 +320,16 @@ __host__ __device__ constexpr int passA_tiles(int K, int LPB)
     return passA_tail(K, LPB) ? (K - 1) / LPB : (K + LPB - 1) / LPB;
 }
 
+// w / d from inv, 1 / d within one ulp.
+template <typename T, bool EXACT>
+__device__ __forceinline__ cpx<T> over_k2(cpx<T> w, T d, T inv)
+{
+#pragma clang fp contract(off)
+    const cpx<T> q = mk<T>(w.re * inv, w.im * inv);
+    if constexpr (!EXACT) return q;
+    else return mk<T>(fma(fma(-d, q.re, w.re), inv, q.re), fma(fma(-d, q.im, w.im), inv, q.im));
+}
+
 template <typename T, int NP, int LPB, int V = 0>
 __device__ __forceinline__ void passA_body(int blk, int nblk, cpx<T> *lds,
                                            const cpx<T> *__restrict__ Wsrc,
@@ -374,8 +391,7 @@ __device__ __forceinline__ void passA_body(int blk, int nblk, cpx<T> *lds,
         const int kt = d.K - 1;
         const cpx<T> w0 = Wsrc[run * bt.sW + (size_t)kt * d.KP];
         const T qt = (T)kt;
-        const T inv = recip(qt * qt);
-        const cpx<T> ps = mk<T>(w0.re * inv, w0.im * inv);
+        const cpx<T> ps = over_k2<T, !C::P2>(w0, qt * qt, recip(qt * qt));
         const T a = (f == 0) ? (T)0 : -qt;
         const cpx<T> val = f == 2 ? w0 : mk<T>(-(a * ps.im), a * ps.re);
         cpx<T> *col = (f == 0 ? Gu : f == 1 ? Gv : Gw) + run * bt.sG + kt;
@@ -399,7 +415,7 @@ __device__ __forceinline__ void passA_body(int blk, int nblk, cpx<T> *lds,
                 const cpx<T> w = sel(kept[s], x[s], ps);
                 const T dd = (kx == 0) ? qy * qy : (kyi == 0) ? qx * qx : qx * qx + qy * qy;
                 const T inv = recip(dd == (T)0 ? (T)1 : dd); // one reciprocal per mode
-                ps = sel(kx == 0 && kyi == 0, ps, mk<T>(w.re * inv, w.im * inv));
+                ps = sel(kx == 0 && kyi == 0, ps, over_k2<T, !C::P2>(w, dd, inv));
             }
             const T a = (f == 0) ? qy : -qx;
             v[s] = mk<T>(-(a * ps.im), a * ps.re);
@@ -903,8 +919,9 @@ struct PassCOperands {
 };
 
 // The Shu-Osher stage update of one mode (src/TimeIntegration.F90:156-202)
-// from the step-start value w0, the stage value ws and dW.
-template <typename T>
+// from the step-start value w0, the stage value ws and dW. THIRDS: stage 3 as
+// the reference's sum of thirds; else one division of the sum.
+template <typename T, bool THIRDS>
 __device__ __forceinline__ cpx<T> rk3_update(int stage, T dt, cpx<T> w0v, cpx<T> wsv, cpx<T> dW)
 {
 #pragma clang fp contract(off)
@@ -916,10 +933,27 @@ __device__ __forceinline__ cpx<T> rk3_update(int stage, T dt, cpx<T> w0v, cpx<T>
                      ((T)0.75 * w0v.im + (T)0.25 * wsv.im) + cc * dW.im);
     }
     const T cc = dt * (T)2;
+    if constexpr (THIRDS)
+        return mk<T>((div3(w0v.re) + div3((T)2 * wsv.re)) + div3(cc * dW.re),
+                     (div3(w0v.im) + div3((T)2 * wsv.im)) + div3(cc * dW.im));
     // (w + 2 w2 + 2 dt dW)/3 correctly rounded: a rounded 1/3 multiplier
     // alone would bias |w| by its rounding error every step
     return mk<T>(div3(((w0v.re + (T)2 * wsv.re) + cc * dW.re)),
                  div3(((w0v.im + (T)2 * wsv.im) + cc * dW.im)));
+}
+
+// TransformR2C's division by the grid size.
+template <typename T, int NP>
+__device__ __forceinline__ cpx<T> over_norm(cpx<T> x, const StageArgs &a)
+{
+#pragma clang fp contract(off)
+    if constexpr (sizeof(T) == 8 && !WaveCfg<T, NP>::P2) {
+        bool odd = false;
+        return mk<T>(div_by(x.re, a.norm, a.inv_norm, &odd), div_by(x.im, a.norm, a.inv_norm, &odd));
+    } else {
+        const T r = (T)a.inv_norm;
+        return mk<T>(x.re * r, x.im * r);
+    }
 }
 
 // The RHS, truncation and stage update of half HALF's rows of column kx;
@@ -937,8 +971,7 @@ __device__ __forceinline__ void passC_finish(const cpx<T> (&v)[WaveCfg<T, NP, V>
     constexpr int E = C::E, TG = C::TG, H = NP / 3;
     const T dt = (T)dtd;
     const T qx = (T)kx;
-    const T inv_norm = (T)a.inv_norm; // multiplications instead of the
-                                      // reference's divisions: <= 1 ulp
+    auto normalized = [&](cpx<T> x) { return over_norm<T, NP>(x, a); };
     const int it = LdsMap<TG>::idx(t);
     static_for<0, E / 2>([&](auto iI) {
         constexpr int i = decltype(iI)::value, s = 2 * i + HALF;
@@ -951,15 +984,14 @@ __device__ __forceinline__ void passC_finish(const cpx<T> (&v)[WaveCfg<T, NP, V>
             const bool keep = kx * kx + kyi * kyi <= H * H;
             const cpx<T> o = other[LdsMap<TG>::idx_sum(it, TG * s)]; // j = t + TG s
             const cpx<T> Pr = HALF == 0 ? v[s] : o, Qr = HALF == 0 ? o : v[s];
-            const cpx<T> P = mk<T>(Pr.re * inv_norm, Pr.im * inv_norm);
-            const cpx<T> Q = mk<T>(Qr.re * inv_norm, Qr.im * inv_norm);
+            const cpx<T> P = normalized(Pr), Q = normalized(Qr);
             const cpx<T> du = mk<T>(-(qx * P.im), qx * P.re); // DuDx of (uw)^
             const cpx<T> dv = mk<T>(-(qy * Q.im), qy * Q.re); // DuDy of (vw)^
             const T sn = (T)nu * (qx * qx + qy * qy);
             const cpx<T> wsv = op.ws[i], w0v = op.w0[i];
             cpx<T> dW = mk<T>((-du.re - dv.re) - sn * wsv.re, (-du.im - dv.im) - sn * wsv.im);
             if (forced) dW = mk<T>(dW.re - op.fv[i].re, dW.im - op.fv[i].im); // closure / forcing
-            cpx<T> out = rk3_update<T>(a.stage, dt, w0v, wsv, dW);
+            cpx<T> out = rk3_update<T, !WaveCfg<T, NP, V>::P2>(a.stage, dt, w0v, wsv, dW);
             out = sel(keep, out, mk<T>((T)0, (T)0));
             if (active && op.row[i]) Wout[col + op.c[i]] = out;
         }
@@ -1110,14 +1142,13 @@ __device__ __forceinline__ void passC_tail(int run, cpx<T> *lds_all, const cpx<T
         cpx<T> P = lds_all[0];
 #pragma unroll
         for (int w = 1; w < NW; ++w) P = add(P, lds_all[w]);
-        const T inv_norm = (T)a.inv_norm;
-        P = mk<T>(P.re * inv_norm, P.im * inv_norm);
+        P = over_norm<T, NP>(P, a);
         const T qx = (T)kx;
         const cpx<T> du = mk<T>(-(qx * P.im), qx * P.re); // DuDx of (uw)^
         const T sn = nu * (qx * qx);
         cpx<T> dW = mk<T>((-du.re) - sn * wsv.re, (-du.im) - sn * wsv.im);
         if (Fc) dW = mk<T>(dW.re - fcv.re, dW.im - fcv.im);
-        if (dtd != 0.0) Wout[col] = rk3_update<T>(a.stage, (T)dtd, w0v, wsv, dW);
+        if (dtd != 0.0) Wout[col] = rk3_update<T, !WaveCfg<T, NP, V>::P2>(a.stage, (T)dtd, w0v, wsv, dW);
     }
     for (int c = 1 + threadIdx.x; c <= d.N; c += NT) Wout[col + c] = mk<T>((T)0, (T)0);
 }

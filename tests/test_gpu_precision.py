@@ -1,5 +1,6 @@
-"""The compiled transforms are as accurate as the runtime plans
-(S2D_GENERIC_KERNELS=1): errors against the exact result, mean over seeds."""
+"""The compiled transforms and the fused step's compiled kernels of the sizes
+96 * 2^k are as accurate as the runtime plans (S2D_GENERIC_KERNELS=1): errors
+against the exact result, mean over seeds."""
 import math
 import os
 
@@ -54,4 +55,57 @@ def test_round_trip(nx, ny, prec):
         s.close()
         err.append(math.exp(np.mean(np.log(e))))
     print(f"[precision] {nx}x{ny} prec={prec} plans {err[0]:.3e} compiled {err[1]:.3e}", flush=True)
+    assert err[1] <= BAR * err[0]
+
+
+class Reference:
+    """The RK3 step of the padded grid in 80 bits."""
+
+    def __init__(self, s):
+        self.shape = (s.nyG, s.nxG)
+        kx, ky = s.kx[None, :].astype(np.longdouble), s.ky[:, None].astype(np.longdouble)
+        self.k2 = kx * kx + ky * ky
+        self.inv_k2 = np.where(self.k2 > 0, 1 / np.maximum(self.k2, 1), 0)
+        self.kept = self.k2 <= (s.nx // 2) ** 2
+        self.dx = np.where(kx == s.nxG // 2, 0, kx)
+        self.dy = np.where(ky == s.nyG // 2, 0, ky)
+
+    def rhs(self, w, nu):
+        psi = w * self.inv_k2
+        u, v, om = (np.fft.irfft2(f, s=self.shape, norm="forward")
+                    for f in (1j * self.dy * psi, -1j * self.dx * psi, w))
+        p, q = (np.fft.rfft2(f, norm="forward") * self.kept for f in (u * om, v * om))
+        return -(1j * self.dx * p + 1j * self.dy * q) - nu * self.k2 * w
+
+    def step(self, w, nu, dt):
+        w, nu, dt = w.astype(np.clongdouble), np.longdouble(nu), np.longdouble(dt)
+        a = (w + dt * self.rhs(w, nu)) * self.kept
+        a = (0.75 * w + 0.25 * a + 0.25 * dt * self.rhs(a, nu)) * self.kept
+        return (w / 3 + 2 * a / 3 + 2 * dt / 3 * self.rhs(a, nu)) * self.kept
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("N", [96, 192, 384])
+def test_step(N, prec):
+    """One fixed step of turbulence of kinetic energy 1/2."""
+    nu, dt = 1e-4, 0.2 * math.pi / N
+    ref, err = {}, []
+    for generic in (True, False):
+        s = make(N, N, prec, generic)
+        r = Reference(s)
+        e = []
+        for seed in SEEDS:
+            w = spectrum(s, seed, 4.0 + 1.5 * seed)
+            w *= math.sqrt(0.5 / (np.abs(w) ** 2 * r.inv_k2).sum())
+            if prec == FP32:
+                w = w.astype(np.complex64).astype(complex)
+            if seed not in ref:
+                ref[seed] = r.step(w, nu, dt)
+            s.set_field("w", w.view(np.float64))
+            s.ComputePsi()
+            s.rk3_step(nu, dt)
+            e.append(rel(s.cview(s.get_field("w")), ref[seed]))
+        s.close()
+        err.append(math.exp(np.mean(np.log(e))))
+    print(f"[precision] step {N} prec={prec} plans {err[0]:.3e} compiled {err[1]:.3e}", flush=True)
     assert err[1] <= BAR * err[0]
