@@ -281,18 +281,22 @@ int s2d_set_taylor_green(s2d_ctx *ctx);
  * context's padded size (index 0 is the default; the single-run sizes
  * Np = 768, 1536, 3072 carry alternatives: the other twiddle batching, the
  * other pass B row pairing and, in FP32, other elements per lane or
- * twiddles for passes A and C), and whether calls of a few steps replay one
- * captured step (hipGraph; longer ones launch ahead of the device).
+ * twiddles for passes A and C), and which calls replay one captured step
+ * (hipGraph) instead of launching their steps' kernels ahead of the device.
  * Every variant computes the same mathematics; results differ at rounding
  * level only. */
 typedef struct s2d_schedule {
     int pass_a, pass_b, pass_c; /* variant index of each pass */
-    int step_graph;             /* 1: short calls replay a captured step */
+    int step_graph;             /* S2D_STEP_*: the calls that replay a captured step */
     double step_us;             /* s2d_tune: measured microseconds per step */
     double default_us;          /* s2d_tune: the default schedule's, eager */
     int candidates, rejected;   /* s2d_tune: schedules timed / failing the check */
     int from_cache;             /* s2d_tune: 1 when read from the cache */
 } s2d_schedule;
+#define S2D_STEP_LAUNCH 0       /* none */
+#define S2D_STEP_REPLAY 1       /* all (any other value too) */
+#define S2D_STEP_DEFAULT 2      /* calls of up to three steps; all of them below N = 96 */
+#define S2D_STEP_REPLAY_SHORT 3 /* calls of up to three steps */
 #define S2D_TUNE_MEASURE 1      /* measure even when the cache has an entry */
 #define S2D_TUNE_CACHE_ONLY 2   /* never measure: the cache's entry or the default */
 /* n[3]: the variants compiled for each pass at this context's size. */
@@ -302,8 +306,9 @@ int s2d_set_schedule(s2d_ctx *ctx, const s2d_schedule *s);
 /* Time every schedule on the context's own buffers from its current state
  * (steps with nu, dt, cfl as in s2d_rk3_steps), reject any whose step
  * differs from the default's by more than rounding (relative L2 of the new
- * state 1e-12 in FP64, 1e-5 in FP32), set the fastest and restore the state
- * (time and step count included). cache: a JSON-lines file (NULL or "": none)
+ * state 1e-12 in FP64, 1e-5 in FP32), set the fastest over eight steps and
+ * restore the state (time and step count included). Where that launches its
+ * steps, single steps decide whether the short calls replay. cache: a JSON-lines file (NULL or "": none)
  * keyed by device, precision and grid; without S2D_TUNE_MEASURE an entry in
  * it is used as is. out (may be NULL) receives the choice. */
 int s2d_tune(s2d_ctx *ctx, double nu, double dt, double cfl, const char *cache, int flags,

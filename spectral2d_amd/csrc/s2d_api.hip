@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdint>
@@ -1288,6 +1289,22 @@ int fused_steps_graphed(s2d_ctx *c, int nsteps, double nu, double dt, double cfl
     return S2D_OK;
 }
 
+// The end of a call of fused steps: the check of the new state and the device
+// scalars, with the call's one wait.
+int finish_steps(s2d_ctx *c, DevScalars *sc)
+{
+    c->ref_stale = true;
+    const size_t n = (size_t)c->K * c->KP;
+    if (c->precision == S2D_FP64)
+        hipLaunchKernelGGL(k_check_finite<double>, dim3(grid_blocks(n, 256)), dim3(256), 0,
+                           c->stream, (const cpx<double> *)c->Wn, n, (long long)n, c->d_sc);
+    else
+        hipLaunchKernelGGL(k_check_finite<float>, dim3(grid_blocks(n, 256)), dim3(256), 0,
+                           c->stream, (const cpx<float> *)c->Wn, n, (long long)n, c->d_sc);
+    S2D_LAUNCHED(c, "k_check_finite");
+    return read_back(c, {{sc, c->d_sc, sizeof(*sc)}});
+}
+
 
 } // namespace
 
@@ -1828,35 +1845,15 @@ int s2d_rk3_steps(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
     }
     S2D_TRY(ensure_compact(c));
     if (nsteps == 0) return sync(c);
-    // Short calls of a single run with the compiled wave kernels replay one
-    // captured step. A replay starts about 10 us sooner than nine launches
-    // do, but leaves about 4.5 us of gap before the next replay (launches that
-    // run ahead of the device leave none), so calls of 4 steps and more launch
-    // them one by one: us per call of 1 / 2 / 8 steps, replayed / launched,
-    // FP64: N = 96 79 / 90, 136 / 144, 474 / 461; N = 512 121 / 129,
-    // 218 / 223, 803 / 785; N = 1024 (10 steps) 1672 / 1627. A step at N = 64
-    // (44 us) is as short as its nine launches take on a slow host (8 steps
-    // 398 / 418, on a fast one 400 / 386) and is always replayed.
-    const bool graphed = c->step_graph_on && c->nruns == 1 &&
-                         (nsteps < 4 || c->g.nxG < 144) &&
+    // a single run with the compiled wave kernels (step_graph.hpp)
+    const bool graphed = step_replays(c->step_graph_set, nsteps, c->g.nxG) && c->nruns == 1 &&
                          (c->precision == S2D_FP64 ? wave_np<double>(c) : wave_np<float>(c)) != 0;
     if (graphed)
         S2D_TRY(S2D_DISPATCH_T(c, fused_steps_graphed, nsteps, nu, dt, cfl));
     else
         S2D_TRY(S2D_DISPATCH_T(c, fused_steps, nsteps, nu, dt, cfl));
-    c->ref_stale = true;
-    {
-        const size_t n = (size_t)c->K * c->KP;
-        if (c->precision == S2D_FP64)
-            hipLaunchKernelGGL(k_check_finite<double>, dim3(grid_blocks(n, 256)), dim3(256), 0,
-                               c->stream, (const cpx<double> *)c->Wn, n, (long long)n, c->d_sc);
-        else
-            hipLaunchKernelGGL(k_check_finite<float>, dim3(grid_blocks(n, 256)), dim3(256), 0,
-                               c->stream, (const cpx<float> *)c->Wn, n, (long long)n, c->d_sc);
-        S2D_LAUNCHED(c, "k_check_finite");
-    }
     DevScalars sc;
-    S2D_TRY(read_back(c, {{&sc, c->d_sc, sizeof(sc)}}));
+    S2D_TRY(finish_steps(c, &sc));
     double vmax;
     std::memcpy(&vmax, &sc.vmax_bits, sizeof(double));
     if (sc.bad || !(vmax == vmax) || vmax > 1.0e300)

@@ -8,6 +8,7 @@
 
 #include "fft_block.hpp"
 #include "s2d.h"
+#include "step_graph.hpp"
 
 namespace s2d {
 
@@ -85,12 +86,12 @@ struct s2d_ctx {
 
     // schedule of the fused step (s2d_set_schedule / s2d_tune): the variant
     // index of passes A, B, C among those compiled for the padded size, and
-    // whether multi-step calls replay a captured step (hipGraph)
+    // which calls replay a captured step (StepGraph)
     int var[3] = {0, 0, 0};
+    int step_graph_set = s2d::STEP_DEFAULT;
     // page-locked staging of small transfers (stage_bytes), each used up
     // before its call returns; null where it could not be had
     char *stage = nullptr;
-    bool step_graph_on = true;
     hipGraphExec_t step_graph = nullptr;
     double sg_nu = 0.0, sg_dt = 0.0, sg_cfl = 0.0; // the captured step's arguments
     const void *sg_forcing = nullptr;              // its forcing buffer (or null)

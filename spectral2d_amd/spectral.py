@@ -241,7 +241,11 @@ class Spectral2D:
         return {k: getattr(s, k) for k, _ in L.Schedule._fields_}
 
     def set_schedule(self, pass_a=0, pass_b=0, pass_c=0, step_graph=True):
-        s = L.Schedule(pass_a, pass_b, pass_c, int(bool(step_graph)))
+        """step_graph: replay a captured step in every call (True), in none
+        (False), in those of up to three steps (3), or in those and in all
+        below N = 96 (2, a new context's setting)."""
+        g = int(step_graph) if step_graph in (2, 3) else int(bool(step_graph))
+        s = L.Schedule(pass_a, pass_b, pass_c, g)
         self._c(L.lib().s2d_set_schedule(self._h, C.byref(s)))
 
     def tune(self, nu: float, dt: float = 0.0, cfl: float = 0.5, cache: str | None = None,
