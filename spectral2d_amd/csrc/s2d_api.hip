@@ -1238,6 +1238,12 @@ void drop_step_graph(s2d_ctx *c)
 {
     if (c->step_graph) (void)hipGraphExecDestroy(c->step_graph);
     c->step_graph = nullptr;
+    c->sg_args = StepArgs();
+}
+
+StepArgs step_args(const s2d_ctx *c, double nu, double dt, double cfl)
+{
+    return {nu, dt, cfl, c->forcing_on ? c->forcing : nullptr, {c->var[0], c->var[1], c->var[2]}};
 }
 
 // One captured step (hipGraph), replayed: its 9 launches go out in one host
@@ -1247,11 +1253,8 @@ void drop_step_graph(s2d_ctx *c)
 template <typename T>
 int fused_steps_graphed(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
 {
-    const void *forcing = c->forcing_on ? c->forcing : nullptr;
-    const bool fresh = c->step_graph && c->sg_nu == nu && c->sg_dt == dt && c->sg_cfl == cfl &&
-                       c->sg_forcing == forcing && c->sg_var[0] == c->var[0] &&
-                       c->sg_var[1] == c->var[1] && c->sg_var[2] == c->var[2];
-    if (!fresh) {
+    const StepArgs args = step_args(c, nu, dt, cfl);
+    if (!c->step_graph || !(c->sg_args == args)) {
         drop_step_graph(c);
         const bool prof = c->prof_on;
         c->prof_on = false; // no timing events inside the graph
@@ -1272,11 +1275,7 @@ int fused_steps_graphed(s2d_ctx *c, int nsteps, double nu, double dt, double cfl
             c->step_graph = nullptr;
             return fail(c, S2D_ERR_HIP, "hipGraphInstantiate failed: %s", hipGetErrorString(ei));
         }
-        c->sg_nu = nu;
-        c->sg_dt = dt;
-        c->sg_cfl = cfl;
-        c->sg_forcing = forcing;
-        for (int k = 0; k < 3; ++k) c->sg_var[k] = c->var[k];
+        c->sg_args = args;
     }
     for (int st = 0; st < nsteps; ++st) {
         if (c->prof_on && c->prof_step % c->prof_every == 0) {
@@ -1846,8 +1845,13 @@ int s2d_rk3_steps(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
     S2D_TRY(ensure_compact(c));
     if (nsteps == 0) return sync(c);
     // a single run with the compiled wave kernels (step_graph.hpp)
-    const bool graphed = step_replays(c->step_graph_set, nsteps, c->g.nxG) && c->nruns == 1 &&
+    bool graphed = step_replays(c->step_graph_set, nsteps, c->g.nxG) && c->nruns == 1 &&
                          (c->precision == S2D_FP64 ? wave_np<double>(c) : wave_np<float>(c)) != 0;
+    if (graphed) {
+        const StepArgs args = step_args(c, nu, dt, cfl);
+        graphed = step_capture_pays(nsteps, args, c->sg_args, c->sg_last);
+        c->sg_last = args;
+    }
     if (graphed)
         S2D_TRY(S2D_DISPATCH_T(c, fused_steps_graphed, nsteps, nu, dt, cfl));
     else

@@ -93,9 +93,8 @@ struct s2d_ctx {
     // before its call returns; null where it could not be had
     char *stage = nullptr;
     hipGraphExec_t step_graph = nullptr;
-    double sg_nu = 0.0, sg_dt = 0.0, sg_cfl = 0.0; // the captured step's arguments
-    const void *sg_forcing = nullptr;              // its forcing buffer (or null)
-    int sg_var[3] = {0, 0, 0};
+    s2d::StepArgs sg_args; // the captured step's (step_graph not null)
+    s2d::StepArgs sg_last; // the last call's that could replay
 
     // fused compact state
     bool fused = false;

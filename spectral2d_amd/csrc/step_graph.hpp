@@ -31,6 +31,31 @@ inline bool step_replays(int setting, int nsteps, int np)
            (setting == STEP_DEFAULT && np < 144);
 }
 
+// What a captured step has baked in.
+struct StepArgs {
+    double nu = 0.0, dt = 0.0, cfl = 0.0;
+    const void *forcing = nullptr; // its buffer, or null
+    int var[3] = {-1, -1, -1};     // the passes' variants (none yet)
+
+    bool operator==(const StepArgs &o) const
+    {
+        return nu == o.nu && dt == o.dt && cfl == o.cfl && forcing == o.forcing &&
+               var[0] == o.var[0] && var[1] == o.var[1] && var[2] == o.var[2];
+    }
+};
+
+// Whether a call that may replay does: a step captured with its arguments is
+// there, or a capture pays, for four steps or for a call like the last one. A
+// program with another dt at every step (the CFL step of its own making) would
+// capture at every call: N = 64 / 96 / 512 / 1024 FP64 126 / 137 / 172 / 249 us
+// a call, launched 74 / 75 / 108 / 181 (the same dt replayed 63 / 76 / 115 /
+// 194).
+inline bool step_capture_pays(int nsteps, const StepArgs &call, const StepArgs &captured,
+                              const StepArgs &last)
+{
+    return call == captured || call == last || nsteps >= 4;
+}
+
 // The setting a measurement picks: replays of all calls where eight steps take
 // least so, else replays of the short calls where one step with its wait does.
 inline int step_graph_choice(double launch8, double replay8, double launch1, double replay1)

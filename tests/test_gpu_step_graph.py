@@ -30,6 +30,26 @@ def test_settings_give_the_same_bits(N, prec):
         assert np.array_equal(w, out[0])
 
 
+@pytest.mark.parametrize("N,prec", [(64, FP32), (96, FP64), (512, FP64)])
+def test_changing_dt(N, prec):
+    """New, repeated and earlier time steps and viscosities, launched and
+    replayed, in calls of one and more steps."""
+    print(f"[step_graph] changing dt N={N} precision={prec}", flush=True)
+    dt = 0.05 / N
+    out = []
+    for setting in (2, True, False):
+        s = Spectral2D(N, precision=prec)
+        s.set_schedule(step_graph=setting)
+        s.SetTurbulence(9, max(2.0, N / 32), 0.5)
+        for k, f, nu in ((1, 1, 1), (1, 2, 1), (1, 3, 1), (1, 3, 1), (1, 3, 1), (2, 1, 1), (1, 3, 1),
+                         (5, 4, 1), (1, 4, 1), (1, 4, 2), (1, 4, 2), (1, 4, 2)):
+            s.rk3_steps(k, nu * 1e-4, f * dt)
+        out.append(s.get_field("w").copy())
+        assert s.get_time()[1] == 17
+        s.close()
+    assert np.array_equal(out[0], out[2]) and np.array_equal(out[1], out[2])
+
+
 def test_tuned_setting_and_former_cache_lines(tmp_path):
     cache, old = str(tmp_path / "tune.jsonl"), str(tmp_path / "old.jsonl")
     s = Spectral2D(512, precision=FP64)

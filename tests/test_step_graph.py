@@ -29,6 +29,26 @@ int main()
     CHECK(step_graph_choice(1.0, 2.0, 2.0, 1.0) == STEP_REPLAY_SHORT);
     CHECK(step_graph_choice(1.0, 2.0, 1.0, 2.0) == STEP_LAUNCH);
     CHECK(step_graph_choice(1.0, 1e300, 1e300, 1e300) == STEP_LAUNCH); // no graph to replay
+    // a capture pays for a call like the last one or the captured one, or for four steps
+    const StepArgs none;
+    StepArgs a, b;
+    a.nu = 1e-4, a.dt = 1e-3, a.var[0] = a.var[1] = a.var[2] = 0;
+    b = a, b.dt = 2e-3;
+    for (int n = 1; n < 8; ++n) {
+        CHECK(step_capture_pays(n, a, none, none) == (n >= 4));
+        CHECK(step_capture_pays(n, b, none, a) == (n >= 4));
+        CHECK(step_capture_pays(n, b, a, a) == (n >= 4));
+        CHECK(step_capture_pays(n, a, none, a));
+        CHECK(step_capture_pays(n, a, a, b));
+    }
+    for (int k = 0; k < 6; ++k) { // every argument counts
+        b = a;
+        if (k == 0) b.nu = 0.0;
+        else if (k == 1) b.cfl = 0.5;
+        else if (k == 2) b.forcing = &b;
+        else b.var[k - 3] = 1;
+        CHECK(!(a == b) && !step_capture_pays(1, a, b, b));
+    }
     return bad;
 }
 """
