@@ -226,7 +226,7 @@ int s2d_axpby(s2d_ctx *ctx, double a, int x, double b, int y);
  * dW = -N - nu k^2 w - F, with F the kept modes of slot f at the time of
  * the call (frozen until the next s2d_set_forcing). The closure term of a
  * coarse run enters as F = tau_hat. s2d_clear_forcing turns it off.
- * Single-run contexts with the compiled fused kernels only. */
+ * Single-run contexts with the fused step only. */
 int s2d_set_forcing(s2d_ctx *ctx, int f);
 int s2d_clear_forcing(s2d_ctx *ctx);
 /* The closure forcing of a coarse run in one call: the state's w and psi

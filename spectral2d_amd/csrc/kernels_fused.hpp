@@ -18,7 +18,7 @@
 //     kx <= N/2. Also the max of |u|+|v| for the CFL step.
 //  C  (per kx column)  forward FFT along y of H_uw, H_vw, then on the kept
 //     modes: /(Np*Np) (TransformR2C), truncation, i kx, i ky, dW =
-//     -N - nu |k|^2 omega_stage, and the Shu-Osher stage update
+//     -N - nu |k|^2 omega_stage (- F, a forcing), and the Shu-Osher stage update
 //     (src/TimeIntegration.F90:156-202), writing the next compact omega.
 // In exact arithmetic this is src/Spectral.F90:396-482 composed with
 // src/TimeIntegration.F90:130-210; the reference's FFT(IFFT(omega)) round
@@ -255,7 +255,7 @@ template <typename T, int E>
 __global__ void k_passC(const cpx<T> *__restrict__ Huw, const cpx<T> *__restrict__ Hvw,
                         const cpx<T> *Wn, const cpx<T> *Wst, cpx<T> *Wout, FusedDims d, FftPlan p,
                         const cpx<T> *__restrict__ tw, const int *__restrict__ trunc_i1,
-                        DevScalars *sc, StageArgs a)
+                        const cpx<T> *__restrict__ forcing, DevScalars *sc, StageArgs a)
 {
 #pragma clang fp contract(off)
     extern __shared__ __align__(16) unsigned char smem[];
@@ -291,6 +291,10 @@ __global__ void k_passC(const cpx<T> *__restrict__ Huw, const cpx<T> *__restrict
             const T sn = (T)a.nu * (qx * qx + qy * qy);
             cpx<T> ws = Wst[col + c];
             cpx<T> dW = mk<T>((-du.re - dv.re) - sn * ws.re, (-du.im - dv.im) - sn * ws.im);
+            if (forcing) { // uniform
+                const cpx<T> f = forcing[col + c];
+                dW = mk<T>(dW.re - f.re, dW.im - f.im);
+            }
             cpx<T> w0 = Wn[col + c];
             if (dtd == 0.0) {
                 out = w0; // a run at its end time keeps its state

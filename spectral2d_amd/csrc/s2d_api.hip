@@ -661,7 +661,8 @@ int launch_passC(s2d_ctx *c, const cpx<T> *Wst, cpx<T> *Wout, const StageArgs &a
     allow_lds(kern, lds);
     launch(c, kern, dim3(d.K), dim3(2 * p.T), lds, (const cpx<T> *)c->H[0],
            (const cpx<T> *)c->H[1], (const cpx<T> *)c->Wn, Wst, Wout, d, p,
-           (const cpx<T> *)c->col.tw, c->d_trunc, c->d_sc, a);
+           (const cpx<T> *)c->col.tw, c->d_trunc,
+           c->forcing_on ? (const cpx<T> *)c->forcing : nullptr, c->d_sc, a);
     S2D_LAUNCHED(c, "k_passC");
     return S2D_OK;
 }
