@@ -1020,10 +1020,11 @@ void wrote(s2d_ctx *c, int f)
     if (f == S2D_FIELD_W) c->compact_stale = true;
 }
 
-// Blocks of the diagnostics' reductions (at most n_red).
+// Blocks of the diagnostics' reductions: at most 512 whatever the batch, so
+// that a run's sums have the same order alone and in any ensemble.
 int diag_blocks(const s2d_ctx *c)
 {
-    return std::min(grid_blocks(nc_of(c), 256), c->n_red);
+    return std::min(grid_blocks(nc_of(c), 256), 512);
 }
 
 // The sums a[5] and a run's scalars as s2d_diagnostics returns them.
@@ -1593,11 +1594,10 @@ int create_ctx(int nx, int ny, int dealias, int precision, int nruns, hipStream_
         c->err = "batched runs need a padded size with compiled kernels (N = 64..2048, powers of 2)";
         return bail(S2D_ERR_UNSUPPORTED);
     }
-    c->n_red = 512 > nruns ? 512 : nruns;
     // the diagnostics' partials and sums of every run, a spectrum's shells
     const size_t nred = std::max((size_t)5 * nruns * (diag_blocks(c) + 1),
                                  2 * (size_t)s2d_spectrum_bins(&c->g));
-    if (hipMalloc(&c->d_red, sizeof(double) * std::max(nred, 6 * (size_t)c->n_red))) {
+    if (hipMalloc(&c->d_red, sizeof(double) * nred)) {
         c->err = "device allocation of reduction buffers failed";
         return bail(S2D_ERR_ALLOC);
     }

@@ -108,7 +108,6 @@ struct s2d_ctx {
     // slots per run, each on a line of its own (kernels_fused_v2.hpp)
     unsigned long long *vslot = nullptr;
     double *d_red = nullptr; // reduction partials
-    int n_red = 0;
     bool ref_stale = false;     // W/PSI slots behind the compact state
     bool compact_stale = true;  // compact state behind the W slot
 
