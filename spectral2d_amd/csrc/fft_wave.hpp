@@ -159,12 +159,13 @@ constexpr double cos15(int a)
 }
 constexpr double sin15(int a) { return cos15(a - 6); }
 
-// What cos(15 a degrees) has beyond its FP64 value where that is +-sqrt(3)/2,
-// else 0: the one constant of radix 12 that is not exact, and FP64 rounds it
-// by 0.45 of its last place.
+// What cos(15 a degrees) has beyond its value in T where that is +-sqrt(3)/2,
+// else 0: the one constant of radix 12 that is not exact. FP64 rounds it by
+// 0.45 of its last place, FP32 by 0.26. (long double is double on the device.)
+template <typename T>
 constexpr double cos15_low(int a)
 {
-    constexpr double low = 5.01754211090345140e-17; // (long double is double on the device)
+    constexpr double low = sizeof(T) == 8 ? 5.01754211090345140e-17 : kCos15[2] - (double)(float)kCos15[2];
     const double c = cos15(a);
     return c == kCos15[2] ? low : c == -kCos15[2] ? -low : 0.0;
 }
@@ -172,12 +173,14 @@ constexpr double cos15_low(int a)
 // x * exp(D i 2 pi e / N) for compile-time e and N | 24 (D = -1 forward,
 // +1 inverse): multiples of a quarter turn are exact swaps and negations,
 // the rest one complex product with constants.
-// ACC (FP64): sqrt(3)/2 in two terms, one FMA more. As a single constant in
-// every pass its rounding adds up: error of a transform of length 144 / 1152
+// ACC: sqrt(3)/2 in two terms, one FMA more. As a single constant in every
+// pass its rounding adds up: FP64 error of a transform of length 144 / 1152
 // and back 2.83e-16 / 3.07e-16, in two terms here and in radix 3 2.36e-16 /
 // 2.70e-16 (the runtime plans, whose table twiddles all round differently,
-// 2.57e-16 / 2.86e-16); IntegrateOneStep at 96 / 768 / 1024 97 -> 101, 238 ->
-// 242 and 334 -> 336 us.
+// 2.57e-16 / 2.86e-16); an FP32 IntegrateOneStep at 48 / 192 2.18e-7 / 2.63e-7
+// and 1.88e-7 / 1.98e-7 (plans 2.10e-7 / 2.78e-7). FP64 IntegrateOneStep at
+// 96 / 768 / 1024 97 -> 101, 238 -> 242 and 334 -> 336 us, FP32 at 1024
+// 219 -> 221.
 template <typename T, int D, int N, int e, bool ACC = false>
 __device__ __forceinline__ cpx<T> twiddle_const(cpx<T> x)
 {
@@ -192,12 +195,12 @@ __device__ __forceinline__ cpx<T> twiddle_const(cpx<T> x)
         return sg > 0 ? mk<T>(-x.im, x.re) : mk<T>(x.im, -x.re);
     } else {
         constexpr T c = (T)cos15(a), sn = (T)(D * sin15(a));
-        if constexpr (ACC && sizeof(T) == 8 && cos15_low(a) != 0.0) {
-            constexpr T cl = (T)cos15_low(a);
+        if constexpr (ACC && cos15_low<T>(a) != 0.0) {
+            constexpr T cl = (T)cos15_low<T>(a);
             return mk<T>(fma(x.re, c, fma(x.re, cl, -(x.im * sn))),
                          fma(x.im, c, fma(x.im, cl, x.re * sn)));
-        } else if constexpr (ACC && sizeof(T) == 8 && cos15_low(a - 6) != 0.0) {
-            constexpr T sl = (T)(D * cos15_low(a - 6));
+        } else if constexpr (ACC && cos15_low<T>(a - 6) != 0.0) {
+            constexpr T sl = (T)(D * cos15_low<T>(a - 6));
             return mk<T>(fma(-x.im, sn, fma(-x.im, sl, x.re * c)),
                          fma(x.re, sn, fma(x.re, sl, x.im * c)));
         } else {
@@ -207,16 +210,16 @@ __device__ __forceinline__ cpx<T> twiddle_const(cpx<T> x)
 }
 
 // Radix 3 with sqrt(3)/2 in two terms (see twiddle_const).
-template <int D>
-__device__ __forceinline__ void dft3_acc(cpx<double> *a)
+template <typename T, int D>
+__device__ __forceinline__ void dft3_acc(cpx<T> *a)
 {
-    constexpr double h = D < 0 ? cos15(2) : -cos15(2), l = D < 0 ? cos15_low(2) : -cos15_low(2);
-    const cpx<double> t1 = add(a[1], a[2]), q = sub(a[1], a[2]);
-    const cpx<double> t2 = mk(a[0].re - 0.5 * t1.re, a[0].im - 0.5 * t1.im);
-    const cpx<double> t3 = mk(fma(q.re, h, q.re * l), fma(q.im, h, q.im * l));
+    constexpr T h = (T)(-D * cos15(2)), l = (T)(-D * cos15_low<T>(2));
+    const cpx<T> t1 = add(a[1], a[2]), q = sub(a[1], a[2]);
+    const cpx<T> t2 = mk<T>(a[0].re - (T)0.5 * t1.re, a[0].im - (T)0.5 * t1.im);
+    const cpx<T> t3 = mk<T>(fma(q.re, h, q.re * l), fma(q.im, h, q.im * l));
     a[0] = add(a[0], t1);
-    a[1] = mk(t2.re + t3.im, t2.im - t3.re);
-    a[2] = mk(t2.re - t3.im, t2.im + t3.re);
+    a[1] = mk<T>(t2.re + t3.im, t2.im - t3.re);
+    a[2] = mk<T>(t2.re - t3.im, t2.im + t3.re);
 }
 
 // In-register DFT of compile-time size N on a[0..N-1] (natural order in and
@@ -225,8 +228,8 @@ __device__ __forceinline__ void dft3_acc(cpx<double> *a)
 template <typename T, int N, int D, bool ACC = false>
 __device__ __forceinline__ void dft_ct(cpx<T> *a)
 {
-    if constexpr (ACC && sizeof(T) == 8 && N == 3) {
-        dft3_acc<D>(a);
+    if constexpr (ACC && N == 3) {
+        dft3_acc<T, D>(a);
     } else if constexpr (N == 2 || N == 3 || N == 4 || N == 8) {
         dft<T, N, D>(a);
     } else {
@@ -278,8 +281,8 @@ constexpr int early_tw_offset()
 // loads wait once per pass; batched ones hold registers for the whole
 // transform.
 constexpr int TW_EARLY = 1, TW_FINAL = 2, TW_ALL = 3, TW_FINAL_POW = 4;
-// bit 3: the constant twiddles inside the butterflies to more than FP64
-// (twiddle_const's ACC)
+// bit 3: the constants inside the butterflies to more than T (twiddle_const's
+// ACC)
 constexpr int TW_ACC = 8;
 
 template <typename T, int E, int TG, int PRE = TW_ALL>

@@ -39,13 +39,13 @@ struct CtLen {
 // FP64 the early passes' only (the others as the final pass uses them, from
 // L1). Products of three of them in the final pass's place took 4 % less
 // time, but left a larger error than the runtime plans (4.8e-16 against
-// 4.1e-16 of a 1024^2 IntegrateOneStep). FP64 butterflies take sqrt(3)/2 in
-// two terms (TW_ACC), with which every length is at least as accurate as its
+// 4.1e-16 of a 1024^2 IntegrateOneStep). Butterflies take sqrt(3)/2 in two
+// terms (TW_ACC), with which every length is at least as accurate as its
 // runtime plan.
 template <typename T, int N>
 constexpr int ct_tw()
 {
-    return sizeof(T) == 8 ? TW_EARLY | TW_ACC : TW_ALL;
+    return TW_ACC | (sizeof(T) == 8 ? TW_EARLY : TW_ALL);
 }
 
 constexpr int round_up(int a, int b) { return (a + b - 1) / b * b; }

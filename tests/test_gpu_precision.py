@@ -84,10 +84,9 @@ class Reference:
         return (w / 3 + 2 * a / 3 + 2 * dt / 3 * self.rhs(a, nu)) * self.kept
 
 
-@pytest.mark.parametrize("prec", [FP64, FP32])
-@pytest.mark.parametrize("N", [96, 192, 384])
-def test_step(N, prec):
-    """One fixed step of turbulence of kinetic energy 1/2."""
+def step_errors(N, prec, routines):
+    """Error of w after one fixed step of turbulence of kinetic energy 1/2, the
+    fused one or IntegrateOneStep: plans, compiled."""
     nu, dt = 1e-4, 0.2 * math.pi / N
     ref, err = {}, []
     for generic in (True, False):
@@ -103,9 +102,23 @@ def test_step(N, prec):
                 ref[seed] = r.step(w, nu, dt)
             s.set_field("w", w.view(np.float64))
             s.ComputePsi()
-            s.rk3_step(nu, dt)
+            (s.IntegrateOneStep if routines else s.rk3_step)(nu, dt)
             e.append(rel(s.cview(s.get_field("w")), ref[seed]))
         s.close()
         err.append(math.exp(np.mean(np.log(e))))
     print(f"[precision] step {N} prec={prec} plans {err[0]:.3e} compiled {err[1]:.3e}", flush=True)
-    assert err[1] <= BAR * err[0]
+    return err
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("N", [96, 192, 384])
+def test_step(N, prec):
+    plans, compiled = step_errors(N, prec, False)
+    assert compiled <= BAR * plans
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("N", [48, 96, 192])
+def test_integrate_one_step(N, prec):
+    plans, compiled = step_errors(N, prec, True)
+    assert compiled <= BAR * plans
