@@ -71,7 +71,7 @@ KERNEL_TAGS = {"c1": ("k2_passA<", "k2_passB<", "k2_passC<"),
 # the sources the three pass kernels and their launch shapes are compiled from
 PASS_SOURCES = ("fft_block.hpp", "fft_wave.hpp", "kernels_ref.hpp", "kernels_fused.hpp",
                 "kernels_fused_v2.hpp", "kernels_ensemble.hpp", "s2d_internal.hpp",
-                "s2d_ensemble.inc")
+                "s2d_ensemble.inc", "exact_div.hpp")
 
 
 def kernel_source_hash() -> str:

@@ -152,9 +152,10 @@ int s2d_compute_vorticity(s2d_ctx *ctx, int u, int v, int w);
 /* ComputeRHS, src/Spectral.F90:396-482 (overwrites u, v; round-trips w). */
 int s2d_compute_rhs(s2d_ctx *ctx, double nu, int u, int v, int w, int psi,
                     int dW);
-/* IntegrateOneStep, src/TimeIntegration.F90:130-210, composed literally
- * from the per-routine kernels on slots W, PSI, U, V with scratch WS,
- * PSIS, DW. */
+/* IntegrateOneStep, src/TimeIntegration.F90:130-210, with the routines'
+ * arithmetic (the round trips of w included) on slots W, PSI, U, V with
+ * scratch WS, PSIS, DW: three launches a stage where the grid's lengths have
+ * compiled transforms, else routine by routine. */
 int s2d_integrate_one_step(s2d_ctx *ctx, double nu, double dt);
 
 /* The fused device-resident TVD-RK3 step (same mathematics as

@@ -66,10 +66,9 @@ struct WaveCfg {
     // lines (columns / rows) per block of passes A and B, LPB * TG threads.
     // 3*2^k lanes: three waves per block, so that every block is whole waves
     // (FP32 pass A: six, G rows in segments twice as long; 192 lanes: two
-    // columns, whose LDS two blocks still share a CU). What bounds these
-    // sizes is what bounds their neighbours: latency (one round of blocks) up
-    // to Np = 1152, the 256 MB cache and VALU issue at 2304. FP64 Np = 1152:
-    // 13, 21 and 10 us for A, B and C (26, 35 and 28 MB of algorithmic traffic)
+    // columns, whose LDS two blocks still share a CU). Latency bounds them up
+    // to Np = 1152 (one or two rounds of blocks): FP64 Np = 1152 13.3, 23.5
+    // and 10.7 us for A, B and C (26, 35 and 28 MB of algorithmic traffic)
     // powers of two: 256 lanes a block; up to Np = 384, where that makes 3 to
     // 48 blocks, one wave, which spreads a launch over more CUs (pass B FP64
     // Np = 96 / 192 / 384: 8.0 / 8.4 / 9.5 -> 5.4 / 5.6 / 7.1 us, pass A 5.8 /

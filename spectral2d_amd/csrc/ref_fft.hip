@@ -19,7 +19,7 @@
 // physical-space fields never do. Measured, 1536^2 padded FP64 (18.9 MB a
 // field), us: columns of one field 38 -> 14 forward or inverse, rows 16 -> 10
 // to 13; ComputeRHS 370 -> 105 (velocity 25, rows 36, columns 47 moving 94,
-// 113 and 132 MB); IntegrateOneStep 1291 -> 330.
+// 113 and 132 MB); IntegrateOneStep 1291 -> 337.
 #include <hip/hip_runtime.h>
 
 #include "kernels_fused_v2.hpp"
@@ -224,7 +224,8 @@ struct RhsArgs {
 // (src/Spectral.F90:451-481), and with STAGE 1-3 the Shu-Osher update,
 // ComputePsi and Truncate (see ref_rhs_columns), in the routines' own
 // expression order. One field's column is in flight at a time next to the sum
-// (FP64: a second one, loaded ahead, spills, and costs 10 % more).
+// (FP64: at the lengths 3 2^k stages 0 and 3 keep 2 to 16 registers in scratch;
+// with a second column loaded ahead they took 10 % longer).
 template <typename T, int NY, int STAGE>
 __global__ __launch_bounds__((ColCfg<T, NY>::THR))
 __attribute__((amdgpu_waves_per_eu(2))) void
@@ -490,7 +491,8 @@ k_rhs_rows(cpx<T> *u, cpx<T> *v, cpx<T> *w, int cI, int nin, int nout, int ny,
     RowTw<T, H> gt;
     gt.load(tw, t);
     row_c2r<T, H>(ww, lw, t, w0, slice, gt);
-#pragma unroll 1 // (unrolled, the compiler holds both fields' tables and spills)
+#pragma unroll 1 // (FP64 puts 6 / 10 / 22 / 34 registers in scratch at H = 192 / 384 / 768 /
+                 // 1536; unrolled, holding both fields' tables, 21 / 39 / 70 / 83)
     for (int i = 0; i < 2; ++i) {
         cpx<T> *f = (i == 0 ? u : v) + at;
         row_load<T, H>(x, f, t, nin);

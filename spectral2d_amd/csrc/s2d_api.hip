@@ -915,8 +915,8 @@ int fused_steps_wave(s2d_ctx *c, int nsteps, double nu, double dt, double cfl)
 // Padded sizes with compiled lane-group FFT kernels; 0 when the generic
 // kernels are used (the runtime plans: other 2^a 3^b sizes). The compiled
 // kernels win wherever they exist. Measured per launch, generic / compiled,
-// FP64: Np = 144 pass A 8.2 / 4.9 us, B 35 / 6.5, C 8.2 / 5.4; Np = 1152
-// A 29 / 13, B 82 / 21, C 17 / 10 (the plans' index divisions, twiddle
+// FP64: Np = 144 pass A 8.2 / 5.0 us, B 35 / 7.7, C 8.2 / 6.6; Np = 1152
+// A 29 / 13, B 82 / 23, C 17 / 11 (the plans' index divisions, twiddle
 // loads in every pass and a barrier pair per radix; pass B's two rows per
 // lane group leave Np = 144 nine blocks of one wave).
 template <typename T>

@@ -182,7 +182,7 @@ class Spectral2D:
 
     # ---- TimeIntegration_m (src/TimeIntegration.F90:67-68)
     def IntegrateOneStep(self, nu, dt):
-        """The reference step composed literally from the per-routine kernels."""
+        """The reference step with the routines' arithmetic, on the slots."""
         self._c(L.lib().s2d_integrate_one_step(self._h, float(nu), float(dt)))
 
     def rk3_step(self, nu, dt):
